@@ -5,10 +5,8 @@
 //       (src/codegen.cpp:59-65), the way bench/sweep.cu:180-186 does through
 //       kvf::Registry;
 //   kvf_launch_merge
-//       the log-sum-exp merge alone;
-//   kvf_quantize_place, kvf_append_tokens
-//       the KV append step: quantize fp32 rows on the GPU and scatter them to
-//       their physical rows, bit-exact with runtime/kvf_host.h:72-135,166-184.
+//       the log-sum-exp merge alone.
+// The KV append step's entry points are in kvf_quantize.hip.
 #include "kvf_kernels.hpp"
 
 #include <algorithm>
@@ -65,96 +63,6 @@ std::vector<std::string> &variant_ids() {
     std::sort(ids.begin(), ids.end());
   });
   return ids;
-}
-
-// ---------------------------------------------------------------- quantizer
-template <int FMT>
-__global__ void __launch_bounds__(256)
-quantize_place_kernel(const float *__restrict__ x, long long rows, int d, int group, int Hkv,
-                      int n, int order, int bt, const int *table, int max_blocks,
-                      unsigned char *data, uint32_t *meta, const int *positions) {
-  const int lane = threadIdx.x & 63;
-  const long long row = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (row >= rows) return; // whole wavefronts leave together
-  // bulk: row r is token r % n of head (r / n) % Hkv of sequence r / (n Hkv);
-  // append: row r is head r % Hkv of sequence r / Hkv at token positions[b],
-  // and a position outside the layout writes nothing
-  int t, h, b;
-  if (positions) {
-    h = (int)(row % Hkv);
-    b = (int)(row / Hkv);
-    t = positions[b];
-    if (t < 0 || t >= (bt ? max_blocks * bt : n)) return;
-  } else {
-    t = (int)(row % n);
-    h = (int)((row / n) % Hkv);
-    b = (int)(row / ((long long)n * Hkv));
-  }
-  long long prow;
-  if (bt == 0) {
-    prow = order == ORD_HEAD ? ((long long)b * Hkv + h) * n + t : ((long long)b * n + t) * Hkv + h;
-  } else {
-    const long long page = table[(long long)b * max_blocks + t / bt];
-    const long long base = page * Hkv * bt;
-    prow = order == ORD_HEAD ? base + (long long)h * bt + t % bt
-                             : base + (long long)(t % bt) * Hkv + h;
-  }
-  const float *xr = x + row * d;
-  const int per = d / 64; // elements per lane: column = e*64 + lane
-  if constexpr (FMT == FMT_F16) {
-    for (int e = 0; e < per; ++e) {
-      const int col = e * 64 + lane;
-      const _Float16 hv = (_Float16)xr[col];
-      reinterpret_cast<_Float16 *>(data)[prow * d + col] = hv;
-    }
-    return;
-  } else {
-    const int levels = FMT == FMT_INT8 ? 255 : 15;
-    const int rb = FMT == FMT_INT8 ? d : d / 2;
-    const int gpr = d / group;
-    float xv[2];
-    for (int e = 0; e < per; ++e) xv[e] = xr[e * 64 + lane];
-    // min/max over each group: groups of 32 are lane halves, 64 one slot,
-    // 128 both slots of a 64-wide row pair
-    const int span = group < 64 ? group : 64;
-    float lo[2], hi[2];
-    for (int e = 0; e < per; ++e) {
-      lo[e] = xv[e];
-      hi[e] = xv[e];
-      for (int m = 1; m < span; m <<= 1) {
-        lo[e] = fminf(lo[e], __shfl_xor(lo[e], m));
-        hi[e] = fmaxf(hi[e], __shfl_xor(hi[e], m));
-      }
-    }
-    if (group == 128 && per == 2) {
-      lo[0] = lo[1] = fminf(lo[0], lo[1]);
-      hi[0] = hi[1] = fmaxf(hi[0], hi[1]);
-    }
-    for (int e = 0; e < per; ++e) {
-      const int col = e * 64 + lane;
-      const _Float16 zero_h = (_Float16)lo[e];
-      float scale = __fdiv_rn(hi[e] - lo[e], (float)levels);
-      if (scale <= 0.f) scale = 1.f;
-      const _Float16 scale_h = (_Float16)scale;
-      const float zero = (float)zero_h;
-      const float sc = (float)scale_h;
-      const float qf = roundf(__fdiv_rn(xv[e] - zero, sc)); // half away from zero
-      const int qv = (int)fminf(fmaxf(qf, 0.f), (float)levels);
-      const int gi = col / group;
-      if (col % group == 0) {
-        const uint32_t w = (uint32_t)__builtin_bit_cast(uint16_t, scale_h) |
-                           ((uint32_t)__builtin_bit_cast(uint16_t, zero_h) << 16);
-        meta[prow * gpr + gi] = w;
-      }
-      if constexpr (FMT == FMT_INT8) {
-        data[prow * rb + col] = (unsigned char)qv;
-      } else {
-        const int hi_code = __shfl_down(qv, 1);
-        if ((col & 1) == 0)
-          data[prow * rb + col / 2] = (unsigned char)(qv | (hi_code << 4));
-      }
-    }
-  }
 }
 
 } // namespace
@@ -340,60 +248,6 @@ extern "C" int kvf_variant_count(void) { return (int)variant_ids().size(); }
 extern "C" const char *kvf_variant_id(int i) {
   const auto &ids = variant_ids();
   return (i >= 0 && i < (int)ids.size()) ? ids[i].c_str() : nullptr;
-}
-
-namespace {
-hipError_t quantize_rows(int fmt, int group, int d, const float *x, int B, int Hkv, int n,
-                         const int *positions, int order, int block_tokens,
-                         const int *block_table, int max_blocks, unsigned char *data,
-                         void *meta, hipStream_t st) {
-  if (!x || !data || B < 1 || Hkv < 1 || n < 1 || (d != 64 && d != 128)) return hipErrorInvalidValue;
-  if (order != ORD_HEAD && order != ORD_TOKEN) return hipErrorInvalidValue;
-  if (block_tokens < 0 || (block_tokens > 0 && (!block_table || max_blocks * block_tokens < n)))
-    return hipErrorInvalidValue;
-  if (fmt != FMT_F16) {
-    if (!meta || (group != 32 && group != 64 && group != 128) || group > d) return hipErrorInvalidValue;
-  }
-  const long long rows = (long long)B * Hkv * (positions ? 1 : n);
-  const dim3 block(256);
-  const dim3 grid((unsigned)((rows + 3) / 4));
-  uint32_t *m = static_cast<uint32_t *>(meta);
-  switch (fmt) {
-  case FMT_F16:
-    hipLaunchKernelGGL(quantize_place_kernel<FMT_F16>, grid, block, 0, st, x, rows, d, group, Hkv,
-                       n, order, block_tokens, block_table, max_blocks, data, m, positions);
-    break;
-  case FMT_INT8:
-    hipLaunchKernelGGL(quantize_place_kernel<FMT_INT8>, grid, block, 0, st, x, rows, d, group,
-                       Hkv, n, order, block_tokens, block_table, max_blocks, data, m, positions);
-    break;
-  case FMT_INT4:
-    hipLaunchKernelGGL(quantize_place_kernel<FMT_INT4>, grid, block, 0, st, x, rows, d, group,
-                       Hkv, n, order, block_tokens, block_table, max_blocks, data, m, positions);
-    break;
-  default:
-    return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-} // namespace
-
-extern "C" hipError_t kvf_quantize_place(int fmt, int group, int d, const float *x, int B,
-                                         int Hkv, int n, int order, int block_tokens,
-                                         const int *block_table, int max_blocks,
-                                         unsigned char *data, void *meta, hipStream_t st) {
-  return quantize_rows(fmt, group, d, x, B, Hkv, n, nullptr, order, block_tokens, block_table,
-                       max_blocks, data, meta, st);
-}
-
-extern "C" hipError_t kvf_append_tokens(int fmt, int group, int d, const float *x, int B, int Hkv,
-                                        int n, const int *positions, int order,
-                                        int block_tokens, const int *block_table,
-                                        int max_blocks, unsigned char *data, void *meta,
-                                        hipStream_t st) {
-  if (!positions) return hipErrorInvalidValue;
-  return quantize_rows(fmt, group, d, x, B, Hkv, n, positions, order, block_tokens, block_table,
-                       max_blocks, data, meta, st);
 }
 
 extern "C" const char *kvf_version(void) { return "kvforge-mi355x 0.3 (gfx950, ABI 2)"; }
