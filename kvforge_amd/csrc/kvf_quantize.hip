@@ -32,12 +32,11 @@ struct FastDiv {
 // token's rows of all heads lie side by side, and a head at a time would write
 // every line in Hkv pieces from different workgroups).
 struct Place {
-  uint32_t rows;        // B * Hkv * (n, or 1 when appending)
+  uint32_t rows;        // B * Hkv * n
   int n, Hkv, order, bt, max_blocks;
   FastDiv inner, outer; // sizes of the two inner dimensions of a work item
   FastDiv page;         // bt (1 for contiguous)
   const int *table;
-  const int *positions; // append: sequence b's token; null: tokens 0..n-1
 };
 
 // One step of a minimum / maximum over the lanes of a group: the value of the
@@ -82,6 +81,68 @@ __device__ __forceinline__ uint32_t code_div(float a, float sc, float levels) {
   return (uint32_t)(fminf(fmaxf(__fdiv_rn(a, sc), 0.f), levels) + 0.49999997f);
 }
 
+// Quantizes a row's 8 elements [8c, 8c + 8) and writes them, and the group's
+// (scale, zero) from its first lane, to physical row `prow`. All lanes of a
+// row call it together (the reductions stay inside a row).
+template <int FMT, int D, int GQ>
+__device__ __forceinline__ void put_row(f4u v0, f4u v1, int c, long long prow, unsigned char *data, uint32_t *meta) {
+  constexpr int ROW = D * bits_of<FMT>() / 8;
+  float e[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) e[k] = k < 4 ? v0[k % 4] : v1[k % 4];
+  unsigned char *to = data + prow * ROW + c * (8 * bits_of<FMT>() / 8);
+  if constexpr (FMT == FMT_F16) {
+    u4u w;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      w[k] = __builtin_bit_cast(uint32_t, (half2_t){(_Float16)e[2 * k], (_Float16)e[2 * k + 1]});
+    *reinterpret_cast<u4u *>(to) = w;
+  } else {
+    constexpr float LEVELS = FMT == FMT_INT8 ? 255.f : 15.f;
+    constexpr int LPG = GQ / 8; // lanes per group
+    auto mn = [](float a, float b) { return fminf(a, b); };
+    auto mx = [](float a, float b) { return fmaxf(a, b); };
+    float lo = e[0], hi = e[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) {
+      lo = fminf(lo, e[k]);
+      hi = fmaxf(hi, e[k]);
+    }
+    lo = over_group<LPG>(lo, mn);
+    hi = over_group<LPG>(hi, mx);
+    const _Float16 zero_h = (_Float16)lo;
+    float scale = __fdiv_rn(hi - lo, LEVELS);
+    if (scale <= 0.f) scale = 1.f;
+    const _Float16 scale_h = (_Float16)scale;
+    const float zero = (float)zero_h;
+    const float sc = (float)scale_h;
+    if (c % LPG == 0)
+      meta[prow * (D / GQ) + c / LPG] = (uint32_t)__builtin_bit_cast(uint16_t, scale_h) |
+                                           ((uint32_t)__builtin_bit_cast(uint16_t, zero_h) << 16);
+    uint32_t q[8];
+    if (sc > 0.f && sc < INFINITY && fabsf(zero) < INFINITY) {
+      const float r = __fdiv_rn(1.f, sc);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = code_fast(e[k] - zero, sc, r, LEVELS);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = code_div(e[k] - zero, sc, LEVELS);
+    }
+    if constexpr (FMT == FMT_INT8) {
+      u2u w;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        w[k] = q[4 * k] | q[4 * k + 1] << 8 | q[4 * k + 2] << 16 | q[4 * k + 3] << 24;
+      *reinterpret_cast<u2u *>(to) = w;
+    } else {
+      uint32_t w = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w |= q[k] << (4 * k); // even elements in the low nibble
+      *reinterpret_cast<u1u *>(to) = w;
+    }
+  }
+}
+
 // A wave takes R * 512 / D neighbouring work items; all their loads go out
 // before the first is used. The items' (sequence, head, token) come from one
 // scalar division per load of a wave, its first item's, and a carry per lane
@@ -90,16 +151,13 @@ __device__ __forceinline__ uint32_t code_div(float a, float sc, float levels) {
 // tokens in int8:64, head-major contiguous, 339 -> 68 us (5.0 TB/s read and
 // written, a large copy's 5.2); 4 x 4093 tokens in int4:32, paged token-major,
 // 180 -> 36 us (4.3 TB/s). Before, a wave took one row, a lane single elements
-// with byte stores, and every element one division. Appending one token to
-// each of 4 sequences (16 calls in a graph of 8 layers' steps): the graph
-// 154 -> 126 us.
+// with byte stores, and every element one division.
 template <int FMT, int D, int GQ, int R>
 __global__ void __launch_bounds__(256)
 quantize_place_kernel(const float *__restrict__ x, unsigned char *__restrict__ data, uint32_t *__restrict__ meta,
                       const Place p) {
   constexpr int LPR = D / 8;         // lanes per row
   constexpr int RPW = 64 / LPR;      // rows per wave and load
-  constexpr int ROW = D * bits_of<FMT>() / 8;
   const int lane = threadIdx.x & 63;
   const uint32_t wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane % LPR;          // the lane's elements are [8c, 8c + 8)
@@ -133,28 +191,16 @@ quantize_place_kernel(const float *__restrict__ x, unsigned char *__restrict__ d
       b[j] = p.outer.quot(rest);
       mid = rest - b[j] * p.outer.div;
     }
-    // appending, the inner dimension is the heads and the outer one is 1
-    const bool head_inner = p.positions || p.order != ORD_HEAD;
-    h[j] = head_inner ? in : mid;
-    t[j] = head_inner ? mid : in;
+    h[j] = p.order == ORD_HEAD ? mid : in;
+    t[j] = p.order == ORD_HEAD ? in : mid;
   }
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    // logical row (b Hkv + h) n + t; head-major and appended rows are in that order already
-    const uint32_t src = p.positions || p.order == ORD_HEAD ? item[j] : (b[j] * p.Hkv + h[j]) * p.n + t[j];
+    // logical row (b Hkv + h) n + t; head-major items are in that order already
+    const uint32_t src = p.order == ORD_HEAD ? item[j] : (b[j] * p.Hkv + h[j]) * p.n + t[j];
     const float *xr = x + (long long)src * D + c * 8;
     v[j][0] = *reinterpret_cast<const f4u *>(xr);
     v[j][1] = *reinterpret_cast<const f4u *>(xr + 4);
-  }
-  if (p.positions) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      // a position outside the layout writes nothing
-      const int pos = p.positions[b[j]];
-      const bool in = pos >= 0 && pos < (p.bt ? p.max_blocks * p.bt : p.n);
-      ok[j] = ok[j] && in;
-      t[j] = in ? (uint32_t)pos : 0u;
-    }
   }
   if (p.bt) {
 #pragma unroll
@@ -168,131 +214,133 @@ quantize_place_kernel(const float *__restrict__ x, unsigned char *__restrict__ d
     if (p.bt) {
       const uint32_t in = t[j] - p.page.quot(t[j]) * p.bt;
       prow = (long long)page[j] * (p.Hkv * p.bt) + (p.order == ORD_HEAD ? h[j] * p.bt + in : in * p.Hkv + h[j]);
-    } else if (p.positions) {
-      prow = p.order == ORD_HEAD ? (long long)item[j] * p.n + t[j] : ((long long)b[j] * p.n + t[j]) * p.Hkv + h[j];
     } else {
       prow = item[j];
     }
-    float e[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) e[k] = v[j][k / 4][k % 4];
-    unsigned char *to = data + prow * ROW + c * (8 * bits_of<FMT>() / 8);
-    if constexpr (FMT == FMT_F16) {
-      u4u w;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        w[k] = __builtin_bit_cast(uint32_t, (half2_t){(_Float16)e[2 * k], (_Float16)e[2 * k + 1]});
-      *reinterpret_cast<u4u *>(to) = w;
-    } else {
-      constexpr float LEVELS = FMT == FMT_INT8 ? 255.f : 15.f;
-      constexpr int LPG = GQ / 8; // lanes per group
-      auto mn = [](float a, float b) { return fminf(a, b); };
-      auto mx = [](float a, float b) { return fmaxf(a, b); };
-      float lo = e[0], hi = e[0];
-#pragma unroll
-      for (int k = 1; k < 8; ++k) {
-        lo = fminf(lo, e[k]);
-        hi = fmaxf(hi, e[k]);
-      }
-      lo = over_group<LPG>(lo, mn);
-      hi = over_group<LPG>(hi, mx);
-      const _Float16 zero_h = (_Float16)lo;
-      float scale = __fdiv_rn(hi - lo, LEVELS);
-      if (scale <= 0.f) scale = 1.f;
-      const _Float16 scale_h = (_Float16)scale;
-      const float zero = (float)zero_h;
-      const float sc = (float)scale_h;
-      if (c % LPG == 0)
-        meta[prow * (D / GQ) + c / LPG] = (uint32_t)__builtin_bit_cast(uint16_t, scale_h) |
-                                             ((uint32_t)__builtin_bit_cast(uint16_t, zero_h) << 16);
-      uint32_t q[8];
-      if (sc > 0.f && sc < INFINITY && fabsf(zero) < INFINITY) {
-        const float r = __fdiv_rn(1.f, sc);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) q[k] = code_fast(e[k] - zero, sc, r, LEVELS);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) q[k] = code_div(e[k] - zero, sc, LEVELS);
-      }
-      if constexpr (FMT == FMT_INT8) {
-        u2u w;
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-          w[k] = q[4 * k] | q[4 * k + 1] << 8 | q[4 * k + 2] << 16 | q[4 * k + 3] << 24;
-        *reinterpret_cast<u2u *>(to) = w;
-      } else {
-        uint32_t w = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) w |= q[k] << (4 * k); // even elements in the low nibble
-        *reinterpret_cast<u1u *>(to) = w;
-      }
-    }
+    put_row<FMT, D, GQ>(v[j][0], v[j][1], c, prow, data, meta);
   }
 }
 
+// One token per sequence: a workgroup is one wave on 64 * 8 / D neighbouring
+// heads of sequence blockIdx.y (and y + 65535, ...). A handful of rows: nothing
+// but the chain argument -> position -> page id -> store bounds it, so the
+// arguments are 14 dwords that arrive preloaded, the rows' loads go out ahead of
+// the chain, and position and page are scalar. (Captured steps of 8 layers for 4
+// sequences, 16 calls beside 16 other kernels: 118.3 -> 114.7 us a graph against
+// appending through the kernel above.)
 template <int FMT, int D, int GQ>
-hipError_t launch_quantize(const float *x, unsigned char *data, uint32_t *meta, const Place &p, hipStream_t st) {
+__global__ void __launch_bounds__(64)
+append_kernel(const float *__restrict__ x, const int *__restrict__ positions, const int *__restrict__ table,
+              unsigned char *__restrict__ data, uint32_t *__restrict__ meta, const int Hkv, const int limit,
+              const uint32_t bt_order, const int max_blocks, const int B) {
+  constexpr int LPR = D / 8;
+  const int c = threadIdx.x % LPR;
+  const int h = blockIdx.x * (64 / LPR) + threadIdx.x / LPR;
+  const uint32_t bt = bt_order & 0x7fffffffu;
+  const bool head_major = !(bt_order >> 31);
+  int b = blockIdx.y; // the grid has no y past B
+  do {
+    const float *xr = x + ((long long)b * Hkv + min(h, Hkv - 1)) * D + c * 8;
+    const f4u v0 = *reinterpret_cast<const f4u *>(xr), v1 = *reinterpret_cast<const f4u *>(xr + 4);
+    const int pos = positions[b];
+    // a position outside the layout writes nothing (no branch: one would hold
+    // back the rows' loads until the position is there)
+    const bool ok = pos >= 0 && pos < limit;
+    const uint32_t t = ok ? (uint32_t)pos : 0u;
+    long long prow;
+    if (bt) {
+      uint32_t blk, in;
+      if ((bt & (bt - 1)) == 0) {
+        blk = t >> __builtin_ctz(bt);
+        in = t & (bt - 1);
+      } else {
+        blk = t / bt;
+        in = t - blk * bt;
+      }
+      const long long base = (long long)table[(long long)b * max_blocks + blk] * ((long long)Hkv * bt);
+      prow = base + (head_major ? (long long)h * bt + in : (long long)in * Hkv + h);
+    } else {
+      prow = head_major ? ((long long)b * Hkv + h) * limit + t : ((long long)b * limit + t) * Hkv + h;
+    }
+    if (ok && h < Hkv) put_row<FMT, D, GQ>(v0, v1, c, prow, data, meta);
+    b += 65535;
+  } while (b < B);
+}
+
+// What a call names: fmt, group, rows and layout (positions: one token per
+// sequence).
+struct Call {
+  int fmt, group;
+  const float *x;
+  int B, Hkv, n;
+  const int *positions;
+  int order, bt;
+  const int *table;
+  int max_blocks;
+  unsigned char *data;
+  uint32_t *meta;
+};
+
+template <int FMT, int D, int GQ> hipError_t launch_quantize(const Call &q, hipStream_t st) {
+  constexpr uint32_t RPW = 64 / (D / 8);
+  if (q.positions) {
+    const long long limit = q.bt ? (long long)q.max_blocks * q.bt : q.n;
+    const dim3 grid((unsigned)((q.Hkv + RPW - 1) / RPW), (unsigned)std::min(q.B, 65535));
+    const uint32_t bt_order = (uint32_t)q.bt | (q.order == ORD_HEAD ? 0u : 1u << 31);
+    hipLaunchKernelGGL((append_kernel<FMT, D, GQ>), grid, dim3(64), 0, st, q.x, q.positions, q.table, q.data, q.meta,
+                       q.Hkv, (int)std::min(limit, 0x7fffffffLL), bt_order, q.max_blocks, q.B);
+    return hipGetLastError();
+  }
+  Place p;
+  p.rows = (uint32_t)((long long)q.B * q.Hkv * q.n);
+  p.n = q.n;
+  p.Hkv = q.Hkv;
+  p.order = q.order;
+  p.bt = q.bt;
+  p.max_blocks = q.max_blocks;
+  p.inner = FastDiv(q.order == ORD_HEAD ? q.n : q.Hkv);
+  p.outer = FastDiv(q.order == ORD_HEAD ? q.Hkv : q.n);
+  p.page = FastDiv(q.bt ? q.bt : 1);
+  p.table = q.table;
   // 4 loads a lane in flight where the rows give every SIMD of the chip two
   // waves of them; fewer rows spread over more waves
-  constexpr uint32_t RPW = 64 / (D / 8);
   if (p.rows >= 2048u * 4 * RPW) {
     const dim3 grid((p.rows + 16 * RPW - 1) / (16 * RPW));
-    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 4>), grid, dim3(256), 0, st, x, data, meta, p);
+    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 4>), grid, dim3(256), 0, st, q.x, q.data, q.meta, p);
   } else {
     const dim3 grid((p.rows + 4 * RPW - 1) / (4 * RPW));
-    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 1>), grid, dim3(256), 0, st, x, data, meta, p);
+    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 1>), grid, dim3(256), 0, st, q.x, q.data, q.meta, p);
   }
   return hipGetLastError();
 }
 
-template <int D>
-hipError_t launch_format(int fmt, int group, const float *x, unsigned char *data, uint32_t *meta, const Place &p,
-                         hipStream_t st) {
-  switch (fmt) {
+template <int D> hipError_t launch_format(const Call &q, hipStream_t st) {
+  switch (q.fmt) {
   case FMT_F16:
-    return launch_quantize<FMT_F16, D, D>(x, data, meta, p, st);
+    return launch_quantize<FMT_F16, D, D>(q, st);
   case FMT_INT8:
-    if (group == 32) return launch_quantize<FMT_INT8, D, 32>(x, data, meta, p, st);
-    if (group == 64) return launch_quantize<FMT_INT8, D, 64>(x, data, meta, p, st);
-    return launch_quantize<FMT_INT8, D, D>(x, data, meta, p, st);
+    if (q.group == 32) return launch_quantize<FMT_INT8, D, 32>(q, st);
+    if (q.group == 64) return launch_quantize<FMT_INT8, D, 64>(q, st);
+    return launch_quantize<FMT_INT8, D, D>(q, st);
   case FMT_INT4:
-    if (group == 32) return launch_quantize<FMT_INT4, D, 32>(x, data, meta, p, st);
-    if (group == 64) return launch_quantize<FMT_INT4, D, 64>(x, data, meta, p, st);
-    return launch_quantize<FMT_INT4, D, D>(x, data, meta, p, st);
+    if (q.group == 32) return launch_quantize<FMT_INT4, D, 32>(q, st);
+    if (q.group == 64) return launch_quantize<FMT_INT4, D, 64>(q, st);
+    return launch_quantize<FMT_INT4, D, D>(q, st);
   default:
     return hipErrorInvalidValue;
   }
 }
 
-hipError_t quantize_rows(int fmt, int group, int d, const float *x, int B, int Hkv, int n,
-                         const int *positions, int order, int block_tokens,
-                         const int *block_table, int max_blocks, unsigned char *data,
-                         void *meta, hipStream_t st) {
-  if (!x || !data || B < 1 || Hkv < 1 || n < 1 || (d != 64 && d != 128)) return hipErrorInvalidValue;
-  if (order != ORD_HEAD && order != ORD_TOKEN) return hipErrorInvalidValue;
-  if (block_tokens < 0 || (block_tokens > 0 && (!block_table || max_blocks * block_tokens < n)))
-    return hipErrorInvalidValue;
-  if (fmt != FMT_F16) {
-    if (!meta || (group != 32 && group != 64 && group != 128) || group > d) return hipErrorInvalidValue;
+hipError_t quantize_rows(const Call &q, int d, hipStream_t st) {
+  if (!q.x || !q.data || q.B < 1 || q.Hkv < 1 || q.n < 1 || (d != 64 && d != 128)) return hipErrorInvalidValue;
+  if (q.order != ORD_HEAD && q.order != ORD_TOKEN) return hipErrorInvalidValue;
+  if (q.bt < 0 || (q.bt > 0 && (!q.table || q.max_blocks * q.bt < q.n))) return hipErrorInvalidValue;
+  if (q.fmt != FMT_F16) {
+    if (!q.meta || (q.group != 32 && q.group != 64 && q.group != 128) || q.group > d) return hipErrorInvalidValue;
   }
-  const long long rows = (long long)B * Hkv * (positions ? 1 : n);
-  // work items are 31-bit (a grid of one row per 64 threads ended at 2^26 rows)
-  if (rows > 0x7fffffffLL) return hipErrorInvalidValue;
-  Place p;
-  p.rows = (uint32_t)rows;
-  p.n = n;
-  p.Hkv = Hkv;
-  p.order = order;
-  p.bt = block_tokens;
-  p.max_blocks = max_blocks;
-  p.inner = FastDiv(positions ? Hkv : order == ORD_HEAD ? n : Hkv);
-  p.outer = FastDiv(positions ? 1 : order == ORD_HEAD ? Hkv : n);
-  p.page = FastDiv(block_tokens ? block_tokens : 1);
-  p.table = block_table;
-  p.positions = positions;
-  uint32_t *m = static_cast<uint32_t *>(meta);
-  return d == 64 ? launch_format<64>(fmt, group, x, data, m, p, st)
-                 : launch_format<128>(fmt, group, x, data, m, p, st);
+  // work items are 31-bit (a kernel of one row per 64 threads ended at 2^26 rows)
+  if ((long long)q.B * q.Hkv * (q.positions ? 1 : q.n) > 0x7fffffffLL) return hipErrorInvalidValue;
+  return d == 64 ? launch_format<64>(q, st) : launch_format<128>(q, st);
 }
 
 } // namespace
@@ -303,8 +351,8 @@ extern "C" hipError_t kvf_quantize_place(int fmt, int group, int d, const float 
                                          int Hkv, int n, int order, int block_tokens,
                                          const int *block_table, int max_blocks,
                                          unsigned char *data, void *meta, hipStream_t st) {
-  return kvf::gfx950::quantize_rows(fmt, group, d, x, B, Hkv, n, nullptr, order, block_tokens, block_table,
-                                    max_blocks, data, meta, st);
+  return kvf::gfx950::quantize_rows({fmt, group, x, B, Hkv, n, nullptr, order, block_tokens, block_table, max_blocks,
+                                     data, static_cast<uint32_t *>(meta)}, d, st);
 }
 
 extern "C" hipError_t kvf_append_tokens(int fmt, int group, int d, const float *x, int B, int Hkv,
@@ -313,6 +361,6 @@ extern "C" hipError_t kvf_append_tokens(int fmt, int group, int d, const float *
                                         int max_blocks, unsigned char *data, void *meta,
                                         hipStream_t st) {
   if (!positions) return hipErrorInvalidValue;
-  return kvf::gfx950::quantize_rows(fmt, group, d, x, B, Hkv, n, positions, order, block_tokens, block_table,
-                                    max_blocks, data, meta, st);
+  return kvf::gfx950::quantize_rows({fmt, group, x, B, Hkv, n, positions, order, block_tokens, block_table, max_blocks,
+                                     data, static_cast<uint32_t *>(meta)}, d, st);
 }
