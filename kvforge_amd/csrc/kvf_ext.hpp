@@ -13,6 +13,18 @@
 namespace kvf {
 namespace gfx950 {
 
+// Ext::flags, the launch's form in one word that reaches the split kernel in
+// a preloaded register (see decode_partial).
+constexpr uint32_t KX_VARLEN = 1;      // per-sequence lengths
+constexpr uint32_t KX_LPT = 2;         // longest first
+constexpr uint32_t KX_Q16 = 4;         // binary16 query
+constexpr uint32_t KX_HGDIV = 8;       // XCD-affine grid over more than one sequence
+constexpr int KX_NX_SHIFT = 4;         // 4 bits: XCDs of an XCD-affine grid, 0 for (splits, head groups, B)
+constexpr int KX_BS_SHIFT = 8;         // 4 bits: Args::block_shift
+constexpr uint32_t KX_GQ1 = 1u << 12;  // one query head per KV head
+constexpr int KX_MB_SHIFT = 13;        // 19 bits: Args::max_blocks, all ones when it is larger
+constexpr uint32_t KX_MB_MAX = (1u << 19) - 1;
+
 // Extension fields beside Args; all null by default.
 struct Ext {
   const int *seq_lens = nullptr; // per-sequence lengths (Args::n is the maximum)
@@ -20,13 +32,6 @@ struct Ext {
   _Float16 *out16 = nullptr;     // binary16 output instead of Args::out
   bool longest_first = false;    // workgroup slots take sequences by decreasing length (B <= 64)
   unsigned *counters = nullptr;  // [B][head groups][KVF_COUNTER_STRIDE] split counters: fused merge
-  // fused step on a 1-D grid: workgroup w runs split (w / nx) / m of head
-  // group w % nx + nx * ((w / nx) % m), m = head groups / nx, so under the
-  // round-robin dispatch of workgroups to a device's nx XCDs every split of a
-  // head group runs on one XCD (the merge is correct wherever they run: it
-  // publishes through the device-coherent level); 0 keeps the (splits, head
-  // groups, B) grid
-  int nx = 0;
   // persistent step: [0] the item queue's claim counter, [KVF_COUNTER_STRIDE]
   // the count of workgroups done (both zero between calls); the grid is then
   // 1-D and `slots` caps it (0: as many workgroups as are resident at once)
@@ -36,6 +41,12 @@ struct Ext {
   // bring it into the instruction cache for the one that does (set by the
   // launcher when the whole grid is resident at once)
   bool dry_merge = false;
+  // set by the launcher from the fields above and Args: the query in the
+  // format that KX_Q16 names, KX_* bits, and the tokens of a split (uniform
+  // lengths)
+  const void *q = nullptr;
+  uint32_t flags = 0;
+  int chunk = 0;
 };
 
 // How a decode step is enqueued: the split kernel alone (partial_only), and

@@ -142,7 +142,7 @@ template <int FMT> constexpr int bits_of() {
 // the lo halves of packed hi/lo rows when all three fit in 64 KiB.
 constexpr int LDS_LIMIT = 65536;
 template <int D, int G> constexpr bool hl_lds_fits(int nw) {
-  return (2 * nw * G * D + nw * G * 3) * 4 <= LDS_LIMIT;
+  return (2 * nw * G * D + nw * G * 4) * 4 <= LDS_LIMIT;
 }
 template <int FMT, int D, int GQ, int G> constexpr size_t combine_lds(int nw);
 
@@ -181,7 +181,7 @@ template <int FMT, int D, int GQ, int G> struct Geo {
 
 template <int FMT, int D, int GQ, int G> constexpr size_t combine_lds(int nw) {
   const bool sl = Geo<FMT, D, GQ, G>::HL && hl_lds_fits<D, G>(nw);
-  return (size_t)(nw * G * (sl ? 2 * D + 3 : D + 3)) * sizeof(float);
+  return (size_t)(nw * G * (sl ? 2 * D + 4 : D + 4)) * sizeof(float);
 }
 
 __device__ __forceinline__ uint32_t perm(uint32_t s0, uint32_t s1, uint32_t sel) {
@@ -230,6 +230,15 @@ template <int G> __device__ __forceinline__ float sum_head_cols(float x) {
   return x;
 }
 
+// Maximum of x over the columns c' == c (mod G) of the lane's row of 16.
+template <int G> __device__ __forceinline__ float max_head_cols(float x) {
+  if constexpr (G <= 1) x = fmaxf(x, ror16<1>(x));
+  if constexpr (G <= 2) x = fmaxf(x, ror16<2>(x));
+  if constexpr (G <= 4) x = fmaxf(x, ror16<4>(x));
+  if constexpr (G <= 8) x = fmaxf(x, ror16<8>(x));
+  return x;
+}
+
 // Raw buffer loads of NB bytes at voffset through descriptor `rs`.
 template <int NB> struct Raw { uint32_t w[NB >= 4 ? NB / 4 : 1]; };
 
@@ -261,6 +270,32 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, long lo
   const uint32_t n = __builtin_amdgcn_readfirstlane(bytes);
   void *ptr = reinterpret_cast<void *>(((uint64_t)hi << 32) | lo);
   return __builtin_amdgcn_make_buffer_rsrc(ptr, 0, (int)n, RSRC_WORD3);
+}
+
+// Device-coherent store of N floats, written through the XCD's L2 (agent-scope
+// atomic stores, 4 or 8 bytes each; the memory takes any 4-byte alignment).
+template <int N> __device__ __forceinline__ void store_through(float *p, const float (&v)[N]) {
+  if constexpr (N == 1) {
+    __hip_atomic_store(p, v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; i += 2)
+      __hip_atomic_store(reinterpret_cast<uint64_t *>(p + i),
+                         (uint64_t)__builtin_bit_cast(uint32_t, v[i]) |
+                             (uint64_t)__builtin_bit_cast(uint32_t, v[i + 1]) << 32,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// Two binary16 high halves of a hi/lo split, as one value that the low halves
+// are then taken from. Without the empty asm the compiler converts twice, once
+// from the rounded product and once fused with it: the two can differ by a
+// binary16 ulp, and where hi and lo sit in different lanes nothing makes up
+// for that (one head in a hundred was off by 3e-4).
+__device__ __forceinline__ half2_t hi_pair(float v0, float v1) {
+  uint32_t w = __builtin_bit_cast(uint32_t, (half2_t){(_Float16)v0, (_Float16)v1});
+  asm("" : "+v"(w));
+  return __builtin_bit_cast(half2_t, w);
 }
 
 // Order in which a lane's binary16 values hold the 8 elements of one k-step.
@@ -300,6 +335,20 @@ template <int I> __device__ __forceinline__ uint32_t quad_bcast(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, I * 0x55, 0xF, 0xF, false);
 }
 
+// Value of head (4r + I) mod G in lane-row r, of an x that every column of a
+// head holds: the head of accumulator row 4r + I. Rows of 4 columns repeat the
+// heads below 4; of 8 heads, quads alternate between the lower and the upper
+// four, and a rotation by 4 brings the other half.
+template <int G, int I> __device__ __forceinline__ float head_of_row(float x) {
+  if constexpr (G == 1) return x;
+  else {
+    const float own = __builtin_bit_cast(float, quad_bcast<I % (G < 4 ? G : 4)>(__builtin_bit_cast(uint32_t, x)));
+    if constexpr (G <= 4) return own;
+    const float other = ror16<4>(own);
+    return ((threadIdx.x >> 2) ^ (threadIdx.x >> 4)) & 1 ? other : own;
+  }
+}
+
 // Calls f(std::integral_constant<int, i>) for i = 0 .. N-1.
 template <int N, int I = 0, class F> __device__ __forceinline__ void static_for(F &&f) {
   if constexpr (I < N) {
@@ -337,6 +386,13 @@ __device__ __forceinline__ int longest_first(const int *lens, int B, int k, int 
   return idx;
 }
 
+// A value the compiler sees nothing of: inside a branch, what only that branch
+// uses is then not computed (a field of Args not loaded) ahead of it.
+__device__ __forceinline__ int opaque(int v) {
+  asm("" : "+s"(v));
+  return v;
+}
+
 // One work item of the split kernel: split `split` of head group `hb` of
 // sequence slot `b` (a sequence index, or its rank by length with
 // Ext::longest_first). With Ext::queue (decode_persistent), thread 0 claims
@@ -372,11 +428,11 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   const int c = lane & 15;
 
   const int gy = G > 1 ? a.Hkv : a.H; // head groups per sequence
-  const int gq = a.H / a.Hkv;
-  const int hkv = G > 1 ? hb : hb / gq;
+  int hkv = hb;
+  if (G == 1 && !(x.flags & KX_GQ1)) hkv = hb / (a.H / a.Hkv);
 
-  // The split's tiles: with uniform lengths a contiguous chunk, tokens
-  // [t0, t1) (runtime/kvf_kernels.cuh:147-150). With per-sequence lengths:
+  // The split's tiles: with uniform lengths a contiguous chunk of Ext::chunk
+  // tokens, [t0, t1) (see uniform_chunk). With per-sequence lengths:
   // - paged: every S-th tile, tiles split, split + S, ... below the
   //   sequence's length, so the tiles and their page ids are known before the
   //   length arrives;
@@ -387,9 +443,9 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   //   log-uniform batch of 16 sequences took 127 us against 108 us in chunks.
   // Tile j of the split (j = wave + nw * k for a wave's k-th) starts at token
   // (tile0 + tstep * j) * TT.
-  const bool varlen = x.seq_lens != nullptr;
+  const bool varlen = (x.flags & KX_VARLEN) != 0;
   const bool strided = varlen && PAGED;
-  const bool lpt = varlen && x.longest_first && a.B > 1 && a.B <= 64;
+  const bool lpt = (x.flags & KX_LPT) != 0;
   int len = a.n;
   int t0 = 0, t1 = 0, n_tiles = 0, nk = 0;
   int tile0 = strided ? split : 0;
@@ -412,6 +468,19 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       vpages = pg;
     }
   };
+  // their first rows in the layout, from the page ids (32 bits: a row is at
+  // least 72 bytes of payload and metadata, so 2^32 of them do not fit the
+  // memory); one vector computation for 32 tiles
+  uint32_t vrow = 0;
+  auto rows_of_pages = [&](int kb32) __attribute__((always_inline)) {
+    if constexpr (PAGED) {
+      const int kk = kb32 + (lane >> 1);
+      const uint32_t t = ((uint32_t)tile0 + (uint32_t)tstep * (uint32_t)(wave + nw * kk)) * TT + (lane & 1) * SUB;
+      const uint32_t in = t & ((1u << bs) - 1);
+      const uint32_t base = (uint32_t)vpages * ((uint32_t)a.Hkv << bs);
+      vrow = base + (ORD == ORD_HEAD ? ((uint32_t)hkv << bs) + in : in * (uint32_t)a.Hkv + (uint32_t)hkv);
+    }
+  };
   // per-sequence lengths in index order: the first page ids go out before the
   // length is loaded, and the empty asm keeps the compiler from issuing the
   // length's scalar load first (a scalar load's wait covers every scalar load
@@ -424,14 +493,15 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   if (varlen) {
     if (lpt) b = longest_first(x.seq_lens, a.B, b, len);
     else len = x.seq_lens[b];
+    len = max(len, 0); // (a negative length is an empty sequence)
   }
   if (strided) {
     t1 = len;
     const int tt = (len + TT - 1) / TT;
-    n_tiles = tt > split ? (tt - split + a.splits - 1) / a.splits : 0;
+    n_tiles = tt > split ? (int)((unsigned)(tt - split + a.splits - 1) / (unsigned)a.splits) : 0;
   } else {
-    const int per = (len + a.splits - 1) / a.splits;
-    const int chunk = varlen ? (per + TT - 1) / TT * TT : per;
+    int chunk = x.chunk;
+    if (varlen) chunk = ((int)((unsigned)(len + a.splits - 1) / (unsigned)a.splits) + TT - 1) / TT * TT;
     t0 = split * chunk;
     t1 = min(len, t0 + chunk);
     tile0 = t0 / TT;
@@ -439,6 +509,31 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   }
   nk = wave < n_tiles ? (n_tiles - wave + nw - 1) / nw : 0; // this wave's tiles
   if (!early_pages) load_pages(0);
+
+  // query loads, through a descriptor over the head group's rows. A lane's 8
+  // elements of a k-step are 32 bytes of fp32 or 16 of binary16: two loads at
+  // offsets scaled by the element size serve both forms without a branch (the
+  // second one's data is not used for binary16); converted to fp32 where the
+  // query is first needed
+  const bool q16 = (x.flags & KX_Q16) != 0;
+  Raw<16> qw[KSTEPS][2];
+  {
+    const int esh = q16 ? 1 : 2; // log2 bytes per element
+    const long long qrow0 = (long long)b * a.H + (G > 1 ? hkv * G : hb); // first head of the group
+    const __amdgpu_buffer_rsrc_t rq = rsrc(x.q, (qrow0 * D) << esh, (uint32_t)(G * D) << esh);
+    const int qh_lane = G > 1 ? c % G : 0;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+#pragma unroll
+      for (int m = 0; m < SPC; ++m) {
+        const int d0 = (qh_lane * D + (j * 4 * CH + r * CH) * 8 / Gm::BITS + 8 * m) << esh;
+        bload<16, 0>(rq, d0, qw[j * SPC + m][0]);
+        bload<16, 0>(rq, d0 + 16, qw[j * SPC + m][1]);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0); // the tiles' addresses come after
+
+  rows_of_pages(0);
 
   // (group, head) pair of column c in pass p; HL packs the hi half in
   // columns 0-7 and the lo half in 8-15, columns beyond the pairs stay zero
@@ -464,45 +559,80 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   for (int p = 0; p < PASSES; ++p)
     mword[p] = ((4 * r + (c & 3)) * tstride * NG + (col_id(p) % COLS) / G) * 4;
 
-
-  // ---- issue all loads of wave-tile k into buf ---------------------------------
+  // ---- issue all loads of the wave's next tile into buf -------------------------
   // Order: both sub-tiles' K, then the (scale, zero) words, then V. Wait counts
   // are in issue order, so a wave can compute a tile's scores and softmax while
   // its V is still arriving.
-  auto issue = [&](Buf &buf, int k) __attribute__((always_inline)) {
-    const bool live = k >= 0 && k < nk;
-    const int tbase = (tile0 + tstep * (wave + nw * k)) * TT;
+  //
+  // A lone wave issues one instruction in four cycles whichever unit it is
+  // for, so the addresses count as much as the arithmetic. Contiguous rows:
+  // four pointers that advance by the wave's step, one descriptor each over
+  // the whole tile, and the tokens left to the end of the range (`left`, kept
+  // at 0 past it: zero-length descriptors), 17 scalar instructions a tile.
+  // Paged rows: the sub-tile's first row comes out of `vrow` by lane. (With
+  // every descriptor worked out from the token index, a tile of int4 d64
+  // token-major rows took 90 instructions of 360 for addresses, and head-major
+  // ones 35.)
+  // Measured with every row in L2, 4096 tokens by one workgroup a head: int4:32
+  // d64 token-major 25.5 -> 23.3 us, int8:64 paged 31.0 -> 28.8 us, int4:32
+  // d128 head-major 28.7 -> 27.3 us.
+  // Descriptors cover the tokens' strides: a token-major one ends up to a
+  // stride past the last row, where no lane's offset points.
+  const int range_end = strided ? len : min(len, (tile0 + n_tiles) * TT);
+  int tnext = (tile0 + tstep * wave) * TT;          // first token of the next tile
+  int knext = 0;
+  int left = nk > 0 ? max(range_end - tnext, 0) : 0;
+  const int step_tokens = tstep * nw * TT;
+  const uint32_t row_step = (uint32_t)(tstride * ROW), meta_step = (uint32_t)(tstride * NG * 4); // bytes a token
+  long long next_row = 0;
+  if constexpr (!PAGED)
+    next_row = ORD == ORD_HEAD ? ((long long)b * a.Hkv + hkv) * a.n + tnext
+                               : ((long long)b * a.n + tnext) * a.Hkv + hkv;
+  const unsigned char *pk = a.k + next_row * ROW, *pv = a.v + next_row * ROW;
+  const unsigned char *pkm = reinterpret_cast<const unsigned char *>(a.k_meta) + next_row * (NG * 4);
+  const unsigned char *pvm = reinterpret_cast<const unsigned char *>(a.v_meta) + next_row * (NG * 4);
+  auto issue = [&](Buf &buf) __attribute__((always_inline)) {
     __amdgpu_buffer_rsrc_t rk[2], rv[2], rkm[2], rvm[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int ts = tbase + s * SUB;
-      long long row0;
-      if constexpr (!PAGED) {
-        row0 = ORD == ORD_HEAD ? ((long long)b * a.Hkv + hkv) * a.n + ts
-                               : ((long long)b * a.n + ts) * a.Hkv + hkv;
-      } else {
-        if (s == 0 && (k & 31) == 0 && k > 0) load_pages(k);
-        const long long page = live ? __builtin_amdgcn_readlane(vpages, 2 * (k & 31) + s) : 0;
-        const int bt = 1 << bs;
-        const long long base = page * a.Hkv * bt;
-        row0 = ORD == ORD_HEAD ? base + (long long)hkv * bt + (ts & (bt - 1))
-                               : base + (long long)(ts & (bt - 1)) * a.Hkv + hkv;
-      }
-      // tokens this sub-tile may read: up to the sequence end
-      const int nv = live ? min(SUB, max(0, len - ts)) : 0;
-      const uint32_t dbytes = nv > 0 ? (uint32_t)((nv - 1) * tstride * ROW + ROW) : 0u;
-      rk[s] = rsrc(a.k, row0 * ROW, dbytes);
-      rv[s] = rsrc(a.v, row0 * ROW, dbytes);
+    int sub_k = 0, sub_m = 0; // offset of the second sub-tile
+    if constexpr (!PAGED) {
+      const uint32_t nv = (uint32_t)min(left, TT);
+      rk[0] = rk[1] = rsrc(pk, 0, nv * row_step);
+      rv[0] = rv[1] = rsrc(pv, 0, nv * row_step);
+      pk += (long long)step_tokens * row_step;
+      pv += (long long)step_tokens * row_step;
       if constexpr (QUANT) {
-        const uint32_t mbytes = nv > 0 ? (uint32_t)(((nv - 1) * tstride + 1) * NG * 4) : 0u;
-        rkm[s] = rsrc(a.k_meta, row0 * NG * 4, mbytes);
-        rvm[s] = rsrc(a.v_meta, row0 * NG * 4, mbytes);
+        rkm[0] = rkm[1] = rsrc(pkm, 0, nv * meta_step);
+        rvm[0] = rvm[1] = rsrc(pvm, 0, nv * meta_step);
+        pkm += (long long)step_tokens * meta_step;
+        pvm += (long long)step_tokens * meta_step;
+      }
+      sub_k = SUB * (int)row_step;
+      sub_m = SUB * (int)meta_step;
+    } else {
+      if ((knext & 31) == 0 && knext > 0) {
+        load_pages(knext);
+        rows_of_pages(knext);
+      }
+      int sub_left = left;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const uint64_t row = (uint32_t)__builtin_amdgcn_readlane((int)vrow, 2 * (knext & 31) + s);
+        const uint32_t nv = (uint32_t)min(sub_left, SUB);
+        rk[s] = rsrc(a.k, (long long)(row * ROW), nv * row_step);
+        rv[s] = rsrc(a.v, (long long)(row * ROW), nv * row_step);
+        if constexpr (QUANT) {
+          rkm[s] = rsrc(a.k_meta, (long long)(row * (NG * 4)), nv * meta_step);
+          rvm[s] = rsrc(a.v_meta, (long long)(row * (NG * 4)), nv * meta_step);
+        }
+        sub_left = max(sub_left - SUB, 0);
       }
     }
+    left = max(left - step_tokens, 0);
+    ++knext;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int j = 0; j < NCH; ++j) bload<CH, cpol_kv<ORD>()>(rk[s], koff + j * 4 * CH, buf.k[s][j]);
+      for (int j = 0; j < NCH; ++j) bload<CH, cpol_kv<ORD>()>(rk[s], koff + (s ? sub_k : 0) + j * 4 * CH, buf.k[s][j]);
     if constexpr (QUANT) {
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -510,9 +640,9 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
 #pragma unroll
           for (int p = 0; p < PASSES; ++p) {
             Raw<4> t;
-            bload<4, cpol_kv<ORD>()>(rkm[s], mword[p], t);
+            bload<4, cpol_kv<ORD>()>(rkm[s], mword[p] + (s ? sub_m : 0), t);
             buf.kmr[s].w[p] = t.w[0];
-            bload<4, cpol_kv<ORD>()>(rvm[s], mword[p], t);
+            bload<4, cpol_kv<ORD>()>(rvm[s], mword[p] + (s ? sub_m : 0), t);
             buf.vmr[s].w[p] = t.w[0];
           }
         } else
@@ -521,9 +651,9 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             Raw<4> t;
-            bload<4, cpol_kv<ORD>()>(rkm[s], moff[p][i], t);
+            bload<4, cpol_kv<ORD>()>(rkm[s], moff[p][i] + (s ? sub_m : 0), t);
             buf.km[p][4 * s + i] = t.w[0];
-            bload<4, cpol_kv<ORD>()>(rvm[s], moff[p][i], t);
+            bload<4, cpol_kv<ORD>()>(rvm[s], moff[p][i] + (s ? sub_m : 0), t);
             buf.vm[p][4 * s + i] = t.w[0];
           }
       }
@@ -531,10 +661,10 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) bload<VB, cpol_kv<ORD>()>(rv[s], voff[i], buf.v[4 * s + i]);
+      for (int i = 0; i < 4; ++i) bload<VB, cpol_kv<ORD>()>(rv[s], voff[i] + (s ? sub_k : 0), buf.v[4 * s + i]);
   };
 
-  // ---- query loads, then the first DEPTH-1 tiles under them ------------------------
+  // ---- the first DEPTH-1 tiles, under the query loads ------------------------------
   // The ring is three named buffers picked by compile-time index, so every
   // access has a constant address and the buffers stay in registers.
   Buf buf0, buf1, buf2;
@@ -544,74 +674,68 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
     else if constexpr (i == 1) return buf1;
     else return buf2;
   };
-  // query loads: both forms through buffer descriptors over the head group's
-  // rows (the form not in use has length 0 and reads zeros), so the load
-  // stream has no branch; converted to fp32 where the query is first needed
-  Raw<16> qf[KSTEPS][2];
-  Raw<16> qh[KSTEPS];
-  {
-    const long long qrow0 = (long long)b * a.H + (G > 1 ? hkv * G : hb); // first head of the group
-    const __amdgpu_buffer_rsrc_t rqf = rsrc(a.q, qrow0 * D * 4, x.q16 ? 0u : (uint32_t)(G * D * 4));
-    const __amdgpu_buffer_rsrc_t rqh = rsrc(x.q16, qrow0 * D * 2, x.q16 ? (uint32_t)(G * D * 2) : 0u);
-    const int qh_lane = G > 1 ? c % G : 0;
-#pragma unroll
-    for (int j = 0; j < NCH; ++j)
-#pragma unroll
-      for (int m = 0; m < SPC; ++m) {
-        const int d0 = qh_lane * D + (j * 4 * CH + r * CH) * 8 / Gm::BITS + 8 * m;
-        bload<16, 0>(rqf, d0 * 4, qf[j * SPC + m][0]);
-        bload<16, 0>(rqf, d0 * 4 + 16, qf[j * SPC + m][1]);
-        bload<16, 0>(rqh, d0 * 2, qh[j * SPC + m]);
-      }
-  }
   static_for<DEPTH - 1>([&](auto Ui) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    issue(ring(Ui), decltype(Ui)::value);
+    issue(ring(Ui));
   });
   __builtin_amdgcn_sched_barrier(0);
 
-  float raw[KSTEPS][8];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    const half8_t h = __builtin_bit_cast(half8_t, (u32x4_t){qh[ks].w[0], qh[ks].w[1], qh[ks].w[2], qh[ks].w[3]});
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      raw[ks][i] = x.q16 ? (float)h[i] : __builtin_bit_cast(float, qf[ks][i / 4].w[i % 4]);
-  }
-
   // ---- query: binary16 hi/lo B operands, zero outside the column's group ----
+  // (scaled once: the prescale and int4's 1/16 are powers of two, so the
+  // halves and the sum are what separate products would give)
+  float raw[KSTEPS][8];
+  if (q16) {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const half8_t h = __builtin_bit_cast(half8_t, qw[ks][0]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) raw[ks][i] = (float)h[i];
+    }
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) raw[ks][i] = __builtin_bit_cast(float, qw[ks][i / 4].w[i % 4]);
+  }
   half8_t qb[PASSES][NQ][KSTEPS];
   float qs[PASSES]; // sum of q' over the column's (group, head), score units
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
     const int cg = (col_id(p) % COLS) / G;
-    float sum = 0.f;
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
 #pragma unroll
       for (int m = 0; m < SPC; ++m) {
         const int ks = j * SPC + m;
         const int dgrp = ((j * 4 * CH + r * CH) * 8 / Gm::BITS + 8 * m) / GRP;
-        const bool mine = col_live && dgrp == cg;
+        const float scale = col_live && dgrp == cg ? a.scale_log2 * QPS : 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float v = mine ? raw[ks][slot_elem<FMT>(i)] * a.scale_log2 : 0.f;
+        for (int i = 0; i < 8; i += 2) {
           // int4: slots 4-7 meet high nibbles entered as code * 16
-          const float vb = FMT == FMT_INT4 && i >= 4 ? v * (QPS / INT4_HI) : v * QPS;
-          const _Float16 hi = (_Float16)vb;
-          const _Float16 lo = (_Float16)(vb - (float)hi);
+          const float sc = FMT == FMT_INT4 && i >= 4 ? scale * (1.f / INT4_HI) : scale;
+          const float v0 = raw[ks][slot_elem<FMT>(i)] * sc, v1 = raw[ks][slot_elem<FMT>(i + 1)] * sc;
+          const half2_t hi = hi_pair(v0, v1);
+          const half2_t lo = {(_Float16)(v0 - (float)hi.x), (_Float16)(v1 - (float)hi.y)};
           if constexpr (HL) {
-            qb[p][0][ks][i] = col_lo ? lo : hi;
+            const half2_t s = col_lo ? lo : hi;
+            qb[p][0][ks][i] = s.x;
+            qb[p][0][ks][i + 1] = s.y;
           } else {
-            qb[p][0][ks][i] = hi;
-            qb[p][NQ - 1][ks][i] = lo;
+            qb[p][0][ks][i] = hi.x;
+            qb[p][0][ks][i + 1] = hi.y;
+            qb[p][NQ - 1][ks][i] = lo.x;
+            qb[p][NQ - 1][ks][i + 1] = lo.y;
           }
-          sum += v;
+          const float back = FMT == FMT_INT4 && i >= 4 ? INT4_HI : 1.f;
+          sum[(i / 2) & 3] = fmaf(v0, back, sum[(i / 2) & 3]);
+          sum[(i / 2) & 3] = fmaf(v1, back, sum[(i / 2) & 3]);
         }
       }
-    sum += xor16(sum);
-    sum += xor32(sum);
-    qs[p] = col_lo ? 0.f : sum / UNIT;
+    float qsum = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    qsum += xor16(qsum);
+    qsum += xor32(qsum);
+    qs[p] = col_lo ? 0.f : qsum * (1.f / (UNIT * QPS)); // both powers of two
   }
 
   // ---- per-lane state ----------------------------------------------------------
@@ -628,59 +752,21 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   float m_true = -INFINITY; // exact max of this lane's scores, score units
   float l_sum = 0.f;
 
-  // ---- consume one tile --------------------------------------------------------
-  auto compute = [&](Buf &buf, int k, auto mask_tag) __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
-    const int tbase = (tile0 + tstep * (wave + nw * k)) * TT;
-    // per-pass (scale, zero) of tokens tau(r, i) for this lane's group
-    uint32_t kmeta[QUANT ? PASSES : 1][8], vmeta[QUANT ? PASSES : 1][8];
-    if constexpr (QMETA) {
-#pragma unroll
-      for (int p = 0; p < PASSES; ++p) {
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          const uint32_t ks = buf.kmr[st].w[p], vs = buf.vmr[st].w[p];
-          kmeta[p][4 * st + 0] = quad_bcast<0>(ks);
-          kmeta[p][4 * st + 1] = quad_bcast<1>(ks);
-          kmeta[p][4 * st + 2] = quad_bcast<2>(ks);
-          kmeta[p][4 * st + 3] = quad_bcast<3>(ks);
-          vmeta[p][4 * st + 0] = quad_bcast<0>(vs);
-          vmeta[p][4 * st + 1] = quad_bcast<1>(vs);
-          vmeta[p][4 * st + 2] = quad_bcast<2>(vs);
-          vmeta[p][4 * st + 3] = quad_bcast<3>(vs);
-        }
-      }
-    } else if constexpr (QUANT) {
-#pragma unroll
-      for (int p = 0; p < PASSES; ++p)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          kmeta[p][i] = buf.km[p][i];
-          vmeta[p][i] = buf.vm[p][i];
-        }
-    }
-    // masked tokens (outside [t0, t1)) carry weight 0; their values are
-    // zeroed too, so a non-finite entry outside the chunk cannot leak in
-    bool ok[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      ok[i] = true;
-      if constexpr (MASK) {
-        const int t = tbase + tau(r, i);
-        ok[i] = t >= t0 && t < t1;
-#pragma unroll
-        for (int w = 0; w < VW; ++w) buf.v[i].w[w] = ok[i] ? buf.v[i].w[w] : 0u;
-        if constexpr (QUANT) {
-#pragma unroll
-          for (int p = 0; p < PASSES; ++p) vmeta[p][i] = ok[i] ? vmeta[p][i] : 0u;
-        }
-      }
-    }
+  // (scale, zero) of token tau(r, i) for the lane's group: loaded, or with
+  // QMETA the word of the quad's lane that loaded that token's
+  auto meta_of = [&](const auto &quad, const auto &own, int p, auto I) __attribute__((always_inline)) {
+    constexpr int i = decltype(I)::value;
+    if constexpr (QMETA) return quad_bcast<i & 3>(quad[i >> 2].w[p]);
+    else return own[p][i];
+  };
 
+  // ---- consume one tile --------------------------------------------------------
+  auto compute = [&](Buf &buf, int k) __attribute__((always_inline)) {
+    const int tbase = (tile0 + tstep * (wave + nw * k)) * TT;
     // ---- scores: QK^T over (group, head) columns, per sub-tile ----------------
     float s[8];
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
+    static_for<2>([&](auto St) __attribute__((always_inline)) {
+      constexpr int st = decltype(St)::value;
       float4_t cq[PASSES];
 #pragma unroll
       for (int p = 0; p < PASSES; ++p) cq[p] = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -719,21 +805,49 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
               cq[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, qb[p][h2][ks], cq[p], 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int i = 4 * st + jj;
+      static_for<4>([&](auto J) __attribute__((always_inline)) {
+        constexpr int jj = decltype(J)::value;
+        constexpr int i = 4 * decltype(St)::value + jj;
         float w = 0.f;
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
           if constexpr (QUANT) {
-            const uint32_t mk = kmeta[p][i];
+            const uint32_t mk = meta_of(buf.kmr, buf.km, p, std::integral_constant<int, i>{});
             w = fmaf(lo_f(mk), cq[p][jj], fmaf(hi_f(mk), qs[p], w));
           } else {
             w += cq[p][jj];
           }
         }
-        w = sum_head_cols<G>(w); // the (group, hi/lo) columns of this head
-        s[i] = (MASK && !ok[i]) ? -INFINITY : w;
+        s[i] = sum_head_cols<G>(w); // the (group, hi/lo) columns of this head
+      });
+    });
+
+    // A tile that reaches outside [t0, t1): the tokens outside carry weight 0,
+    // and their values are zeroed too, so a non-finite entry there cannot leak
+    // in. Wave-uniform, a branch inside the one body that every tile runs: a
+    // body of its own for such tiles made the kernel half as large again and
+    // cost copies of the first tile's registers where the two met.
+    if (tbase < t0 || tbase + TT > t1) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int t = tbase + tau(r, i);
+        const bool ok = t >= t0 && t < t1;
+        s[i] = ok ? s[i] : -INFINITY;
+#pragma unroll
+        for (int w = 0; w < VW; ++w) buf.v[i].w[w] = ok ? buf.v[i].w[w] : 0u;
+        if constexpr (QUANT && !QMETA) {
+#pragma unroll
+          for (int p = 0; p < PASSES; ++p) buf.vm[p][i] = ok ? buf.vm[p][i] : 0u;
+        }
+      }
+      if constexpr (QMETA) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const int t = tbase + st * SUB + 4 * r + (c & 3); // the lane's word
+          const bool ok = t >= t0 && t < t1;
+#pragma unroll
+          for (int p = 0; p < PASSES; ++p) buf.vmr[st].w[p] = ok ? buf.vmr[st].w[p] : 0u;
+        }
       }
     }
 
@@ -742,8 +856,9 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
                              fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
     m_true = fmaxf(m_true, tmax);
     if (__any(tmax > m_run + TAU_S)) { // wave-uniform, rare after the first tile
-      float cand = fmaxf(m_run, tmax);
-      for (int mask = G; mask < 16; mask <<= 1) cand = fmaxf(cand, __shfl_xor(cand, mask));
+      // (lane crossings by DPP and lane swaps: through LDS, the eight of them
+      // were most of a short split's first tile)
+      float cand = max_head_cols<G>(fmaxf(m_run, tmax));
       cand = fmaxf(cand, xor16(cand));
       cand = fmaxf(cand, xor32(cand));
       // the running max moves on a grid of 2^-8 log2 units (rounded up), so
@@ -759,9 +874,8 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       // accumulator row 4r+i belongs to head (4r+i) mod G: take that
       // column's alpha; whole float4 accumulators are scaled, so each keeps
       // its registers (per-element products were moved back at every tile)
-      float4_t a4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a4[i] = __shfl(alpha, 16 * r + ((4 * r + i) & 15));
+      const float4_t a4 = {head_of_row<G, 0>(alpha), head_of_row<G, 1>(alpha), head_of_row<G, 2>(alpha),
+                           head_of_row<G, 3>(alpha)};
 #pragma unroll
       for (int p = 0; p < PASSES; ++p)
 #pragma unroll
@@ -775,33 +889,43 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
     l_sum += ((pj[0] + pj[1]) + (pj[2] + pj[3])) + ((pj[4] + pj[5]) + (pj[6] + pj[7]));
 
     // ---- weights: V scale folded in, binary16 hi/lo -------------------------------
+    // HL: the lo half has its own accumulator rows, so it enters scaled by
+    // 2^11 (it never exceeds the hi half, so this cannot overflow) and stays
+    // out of the binary16 subnormal range; the rows are scaled back where the
+    // wave's result is combined. A lane keeps one of the halves, by a select
+    // of what every lane works out alike: the hi half that a lo column
+    // subtracts has to be the very value its hi column holds.
     half8_t pa[PASSES][NQ];
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float w = pj[i];
+      static_for<4>([&](auto I2) __attribute__((always_inline)) {
+        constexpr int i = 2 * decltype(I2)::value;
+        float w[2] = {pj[i], pj[i + 1]};
         if constexpr (QUANT) {
-          const uint32_t mv = vmeta[p][i];
-          zacc[p] = fmaf(pj[i], fmaf(vmid<FMT>(), lo_f(mv), hi_f(mv)), zacc[p]);
-          w *= lo_f(mv);
+          const uint32_t mv[2] = {meta_of(buf.vmr, buf.vm, p, std::integral_constant<int, i>{}),
+                                  meta_of(buf.vmr, buf.vm, p, std::integral_constant<int, i + 1>{})};
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            zacc[p] = fmaf(pj[i + e], fmaf(vmid<FMT>(), lo_f(mv[e]), hi_f(mv[e])), zacc[p]);
+            w[e] *= lo_f(mv[e]);
+          }
         }
-        w = col_live ? w : 0.f;
-        if constexpr (HL) {
-          const _Float16 hi = (_Float16)w;
-          // the lo half has its own accumulator rows, so it enters scaled by
-          // 2^11 (it never exceeds the hi half, so this cannot overflow) and
-          // stays out of the binary16 subnormal range; the rows are scaled
-          // back where the wave's result is combined
-          const _Float16 lo = (_Float16)((w - (float)hi) * LO_SCALE);
-          pa[p][0][i] = col_lo ? lo : hi;
-        } else {
-          const _Float16 hi = (_Float16)w;
-          const _Float16 lo = (_Float16)(w - (float)hi);
-          pa[p][0][i] = hi;
-          pa[p][NQ - 1][i] = lo;
+        if constexpr (HL && COLS < 8) {
+          w[0] = col_live ? w[0] : 0.f;
+          w[1] = col_live ? w[1] : 0.f;
         }
-      }
+        const half2_t hi = hi_pair(w[0], w[1]);
+        half2_t first = hi;
+        constexpr float scale = HL ? LO_SCALE : 1.f;
+        const half2_t lo = {(_Float16)((w[0] - (float)hi.x) * scale), (_Float16)((w[1] - (float)hi.y) * scale)};
+        if constexpr (HL) first = col_lo ? lo : hi;
+        pa[p][0][i] = first.x;
+        pa[p][0][i + 1] = first.y;
+        if constexpr (!HL) {
+          pa[p][NQ - 1][i] = lo.x;
+          pa[p][NQ - 1][i + 1] = lo.y;
+        }
+      });
     }
 
     // ---- values: B operand = 8 tokens of one dim, PV MFMA ----------------------------
@@ -837,79 +961,35 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   // Every step issues the tile DEPTH-1 ahead and consumes one; tile k sits in
   // ring slot k % DEPTH. Whole rounds of DEPTH steps run with no exit inside a
   // round (the accumulators then stay in their registers across the loop;
-  // early exits between steps made the compiler copy them at every tile),
-  // then up to DEPTH-1 single steps. The last DEPTH-1 tiles are consumed
-  // after the loop without issuing anything (the drain below), so no
-  // zero-length loads are left in flight for the epilogue to wait on.
-  // Masking: the drain holds the split's last tile, the only one that may end
-  // past t1; split tile 0 starts before t0 only when t0 is not a multiple of
-  // the tile, and then (the one case) every step of the loop is masked.
-  // Inside a round the compiler schedules loads and compute freely (barriers
-  // there cost 3 % on int4:32 and 6 % on long variable-length contiguous
-  // batches); the single steps keep each step's loads ahead of its compute.
-  // Binary16 rows with 4 waves and a ring of 2 take the per-step form instead
-  // (an exit test before every step, each step masked only where its tile
-  // crosses [t0, t1)): it compiles to 248 VGPRs against 255 plus 20 AGPRs for
-  // whole rounds, which keeps two 4-wave workgroups per CU (2 % faster at GQA
-  // 32/8 n32768 f16, 10 % on a batch of 16 sequences that needs several
-  // rounds of workgroups); with 8 waves or a ring of 3 it measured slower
-  // (median 1.3-1.8x over the f16 plans of the uniform sweep). (The per-step
-  // loop is written inline below: wrapped in a lambda it compiled to 256
-  // VGPRs plus 86 AGPRs.)
-  constexpr bool PER_STEP = FMT == FMT_F16 && DEPTH == 2 && WPB == 4;
+  // early exits between steps made the compiler copy them at every tile); the
+  // up to DEPTH-1 tiles that are left are already on their way. A round's last
+  // issues may lie past the wave's tiles: zero-length loads, unconditional so
+  // that the wait counts stay static.
+  // One loop and one body for masked and unmasked tiles alike: with a loop for
+  // each, single steps and a drain (eight bodies), the registers of the tile
+  // in flight were copied where the paths met, which waits for all of it
+  // before the second tile's loads go out. Against that: 34 -> 16 KB of code,
+  // 214 -> 186 VGPRs (int8:64 d128 G 4), a one-tile step 4.77 -> 4.43 us,
+  // int4:32 d64 token-major (16 tiles a wave) 23.3 -> 21.6 us, a captured
+  // batch of 4 short sequences 9.8 -> 9.3 us a layer, the rest as before.
   int k = 0;
-  auto stream = [&](auto mask_tag) __attribute__((always_inline)) {
-    while (k + 2 * DEPTH - 1 <= nk) {
-      static_for<DEPTH>([&](auto Ui) __attribute__((always_inline)) {
-        constexpr int s = decltype(Ui)::value;
-        issue(ring(std::integral_constant<int, (s + DEPTH - 1) % DEPTH>{}), k + DEPTH - 1);
-        compute(ring(Ui), k, mask_tag);
-        ++k;
-      });
-    }
-    static_for<DEPTH - 1>([&](auto Ui) __attribute__((always_inline)) {
+  while (k + DEPTH <= nk) {
+    static_for<DEPTH>([&](auto Ui) __attribute__((always_inline)) {
       constexpr int s = decltype(Ui)::value;
-      if (k + DEPTH - 1 < nk) { // a prefix of the steps: once false, k stays put
-        __builtin_amdgcn_sched_barrier(0);
-        issue(ring(std::integral_constant<int, (s + DEPTH - 1) % DEPTH>{}), k + DEPTH - 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(ring(Ui), k, mask_tag);
-        ++k;
-      }
+      issue(ring(std::integral_constant<int, (s + DEPTH - 1) % DEPTH>{}));
+      compute(ring(Ui), k + s);
     });
-  };
-  if constexpr (PER_STEP) {
-    bool streaming = true;
-    while (streaming) {
-      static_for<DEPTH>([&](auto Ui) __attribute__((always_inline)) {
-        constexpr int u = decltype(Ui)::value;
-        if (!streaming) return;
-        if (k + DEPTH - 1 >= nk) {
-          streaming = false;
-          return;
-        }
-        issue(ring(std::integral_constant<int, (u + DEPTH - 1) % DEPTH>{}), k + DEPTH - 1);
-        const int tbase = (tile0 + tstep * (wave + nw * k)) * TT;
-        if (tbase >= t0 && tbase + TT <= t1) compute(ring(Ui), k, std::false_type{});
-        else compute(ring(Ui), k, std::true_type{});
-        ++k;
-      });
-    }
-  } else if (t0 % TT == 0) stream(std::false_type{});
-  else stream(std::true_type{});
+    k += DEPTH;
+  }
   // persistent step: thread 0 claims the workgroup's next item behind the
   // last tiles' loads, so the claim's round trip overlaps the drain
   unsigned claim = 0;
   if constexpr (QUEUE) {
     if (threadIdx.x == 0) claim = __hip_atomic_fetch_add(x.queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  // drain: the tiles still in flight, masked (a full tile computes the same)
-  for (int j = 0; j < DEPTH - 1; ++j, ++k) {
-    if (k >= nk) break;
-    static_for<DEPTH>([&](auto Ui) __attribute__((always_inline)) {
-      if (k % DEPTH == decltype(Ui)::value) compute(ring(Ui), k, std::true_type{});
-    });
-  }
+  static_for<DEPTH - 1>([&](auto Ui) __attribute__((always_inline)) {
+    if (k + decltype(Ui)::value < nk) compute(ring(Ui), k + decltype(Ui)::value);
+  });
 
   // ---- wave result: per head (m_run, l, m_true) and O[head][D] ---------------
   l_sum += xor16(l_sum);
@@ -927,15 +1007,11 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   }
 
   extern __shared__ __attribute__((aligned(16))) float smem[]; // 16 B: the fused merge reads float4
-  // layout: sO[nw][G][D], sM[nw][G][3], then (HL_LDS) sL[nw][G][D]
+  // layout: sO[nw][G][D], sM[nw][G] (m_run, l, m_true, -), then (HL_LDS) sL[nw][G][D]
   float *sO = smem;
-  float *sM = smem + nw * G * D;
-  float *sL = sM + nw * G * 3;
-  if (r == 0 && c < G) {
-    sM[(wave * G + c) * 3 + 0] = fmaf(m_run, UNIT, -WOFF);
-    sM[(wave * G + c) * 3 + 1] = l_sum;
-    sM[(wave * G + c) * 3 + 2] = m_true * UNIT;
-  }
+  float4_t *sM = reinterpret_cast<float4_t *>(smem + nw * G * D);
+  float *sL = smem + nw * G * (D + 4);
+  if (r == 0 && c < G) sM[wave * G + c] = (float4_t){fmaf(m_run, UNIT, -WOFF), l_sum, m_true * UNIT, 0.f};
   const int gdim = (c * EV) / GRP; // group of this lane's V dims
   // With HL, accumulator rows 8-15 (lane-rows 2 and 3) hold the lo halves of
   // rows 0-7: they are stored to their own LDS rows (sL) and the combine adds
@@ -970,44 +1046,53 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   }
   __syncthreads();
 
-  // every LDS read of an output element is issued before any is used: the
-  // waves' (m_run, l, m_true) and partial outputs, then a branch-free
+  // A thread takes VPT neighbouring dims of one head, so the waves' weights
+  // are worked out once for them (one dim at a time, with three reads for a
+  // wave's (m_run, l, m_true), this and the lane crossings through LDS cost a
+  // one-tile step 0.33 us of 5.1 and 32768 tokens 0.4-0.5 us of 16.7-17.0). Every LDS read is issued before any is used:
+  // the waves' (m_run, l, m_true) and partial outputs, then a branch-free
   // log-sum-exp over the waves (a wave with m_run = -inf saw no token and
-  // contributes nothing; all -inf leaves L = O = 0)
-  const int nthreads = nw * 64;
-#pragma unroll
-  for (int idx0 = 0; idx0 < G * D; idx0 += nthreads) {
-    const int idx = idx0 + threadIdx.x;
-    if (G * D % nthreads != 0 && idx >= G * D) break;
+  // contributes nothing; all -inf leaves L = O = 0).
+  constexpr int VPT = G * D >= nw * 64 ? G * D / (nw * 64) : 1; // 1, 2, 4
+  if (G * D >= nw * 64 || threadIdx.x * VPT < G * D) {
+    const int idx = threadIdx.x * VPT;
     const int hh = idx / D, col = idx % D;
-    float mr[nw], lw[nw], mt[nw], ov[nw];
+    float4_t mw[nw];
+    float ov[nw][VPT];
 #pragma unroll
     for (int w2 = 0; w2 < nw; ++w2) {
-      mr[w2] = sM[(w2 * G + hh) * 3 + 0];
-      lw[w2] = sM[(w2 * G + hh) * 3 + 1];
-      mt[w2] = sM[(w2 * G + hh) * 3 + 2];
-      ov[w2] = sO[(w2 * G + hh) * D + col];
-      if constexpr (HL_LDS) ov[w2] += sL[(w2 * G + hh) * D + col];
+      mw[w2] = sM[w2 * G + hh];
+#pragma unroll
+      for (int e = 0; e < VPT; ++e) {
+        ov[w2][e] = sO[(w2 * G + hh) * D + col + e];
+        if constexpr (HL_LDS) ov[w2][e] += sL[(w2 * G + hh) * D + col + e];
+      }
     }
     float M = -INFINITY;
 #pragma unroll
-    for (int w2 = 0; w2 < nw; ++w2) M = fmaxf(M, mt[w2]);
-    float L = 0.f, O = 0.f;
+    for (int w2 = 0; w2 < nw; ++w2) M = fmaxf(M, mw[w2].z);
+    float L = 0.f, O[VPT];
+#pragma unroll
+    for (int e = 0; e < VPT; ++e) O[e] = 0.f;
 #pragma unroll
     for (int w2 = 0; w2 < nw; ++w2) {
-      const bool live = M != -INFINITY && mr[w2] != -INFINITY;
-      const float wgt = live ? __builtin_amdgcn_exp2f(mr[w2] - M) : 0.f;
-      L = live ? fmaf(lw[w2], wgt, L) : L;
-      O = live ? fmaf(ov[w2], wgt, O) : O;
+      const bool live = M != -INFINITY && mw[w2].x != -INFINITY;
+      const float wgt = live ? __builtin_amdgcn_exp2f(mw[w2].x - M) : 0.f;
+      L = live ? fmaf(mw[w2].y, wgt, L) : L;
+#pragma unroll
+      for (int e = 0; e < VPT; ++e) O[e] = live ? fmaf(ov[w2][e], wgt, O[e]) : O[e];
     }
     const int hq = G > 1 ? hkv * G + hh : hb;
     const long long head = (long long)b * a.H + hq;
     if (final_out) {
-      const float res = L > 0.f ? O / L : 0.f;
-      if (x.out16) x.out16[head * D + col] = (_Float16)res;
-      else a.out[head * D + col] = res;
+#pragma unroll
+      for (int e = 0; e < VPT; ++e) {
+        const float res = L > 0.f ? O[e] / L : 0.f;
+        if (x.out16) x.out16[head * D + col + e] = (_Float16)res;
+        else a.out[head * D + col + e] = res;
+      }
     } else {
-      // agent-scope atomic stores: written through to the level every XCD
+      // device-coherent (sc1) stores: written through to the level every XCD
       // sees while the kernel still runs, so the fused step publishes them
       // without an L2 writeback, and in the two-launch step the writeback at
       // the kernel's end has no partials left to flush before the merge
@@ -1015,12 +1100,13 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       // at 32k tokens 18.2 -> 17.6 us and 18.0 -> 17.9 us, int4 at 64k
       // 24.7 -> 24.2 us, a paged batch of 8 sequences 27.8 -> 28.0 us; the
       // split kernel alone 0.1 us longer)
-      float *po = a.part_o + (head * a.splits + split) * D + col;
-      float *pm = a.part_ml + (head * a.splits + split) * 2;
-      __hip_atomic_store(po, O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const long long row = head * a.splits + split;
+      float *po = a.part_o + row * D + col;
+      float *pm = a.part_ml + row * 2;
+      store_through<VPT>(po, O);
       if (col == 0) {
-        __hip_atomic_store(pm, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(pm + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float ml[2] = {M, L};
+        store_through<2>(pm, ml);
       }
     }
   }
@@ -1054,50 +1140,67 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   }
 }
 
-// The split kernel: a workgroup runs the one item its grid position names,
-// (split, head group, sequence) = blockIdx on the 3-D grid, or the XCD-affine
-// order of the fused step's 1-D grid (Ext::nx).
-// Its first arguments repeat the fields the first loads wait for (the grid's
-// XCD count, the sizes, the cache pointers, 14 dwords), ahead of Args and
-// Ext: the kernel translation units are built with kernel-argument
-// preloading of 14 dwords, so these arrive in SGPRs as the wave starts
-// instead of through a load from the argument segment, and the rest of Args
-// and Ext arrives while the first tiles' addresses are formed. The query
-// pointer follows them. (Measured on MI355X, alternating builds, three
-// rounds: the fused step 17.26-17.30 -> 17.01-17.07 us at GQA 32/8, d128,
-// n32768, int8:64; config 3's fused step 28.18-28.19 -> 27.89-27.93 us; the
-// two-launch steps within 0.05 us.)
+// The split kernel: a workgroup runs the one item its grid position names:
+// (split, head group, sequence) = blockIdx on the plain grid. On the fused
+// step's XCD-affine grid (nx, head groups / nx, splits), nx the device's XCDs,
+// it is split z of head group x + nx * y: under the round-robin dispatch of
+// workgroups to XCDs every split of a head group runs on one XCD (the merge is
+// correct wherever they run: it publishes through the device-coherent level).
+//
+// A short step is a chain of round trips, and the argument segment's is the
+// first of them. So everything the first loads' addresses need comes in the
+// leading 14 dwords, ahead of Args and Ext: the kernel translation units are
+// built with kernel-argument preloading of 14 dwords, which arrive in SGPRs as
+// the wave starts. Ext::flags, the KV heads and splits (16 bits each), the
+// token count and the split's chunk (or the lengths' pointer, per-sequence
+// lengths), the four cache pointers, and the query (paged: the page table; the
+// query's pointer then arrives while the page ids are on their way). Fields
+// that only some forms need are read from Args inside an opaque branch: a
+// plain select would load them, and wait, in every form. Grid positions and
+// chunks come divided from the host (four run-time divisions are 0.25 us).
+// Measured on MI355X, back to back, GQA 32/8 d128 int8:64: 128 tokens and one
+// split, a tile for every wave and one kernel, 5.69 -> 5.12 us a step; 32768
+// tokens and 32 splits 17.2-17.5 -> 16.7-17.0 us (with the old query loads,
+// both formats', and run-time divisions against without).
 template <int FMT, int D, int GQ, int G, int U, int ORD, bool PAGED, int WPB>
 __global__ void __launch_bounds__(WPB * 64)
-decode_partial(const int nx, const int n, const int splits, const int H, const int Hkv, const int B,
-               const void *k, const void *v, const void *k_meta, const void *v_meta, const void *q,
-               const Args args, const Ext ext, const int final_out) {
+decode_partial(const uint32_t flags, const uint32_t heads_splits, const void *n_chunk, const void *k, const void *v,
+               const void *k_meta, const void *v_meta, const void *q_or_table, const Args args, const Ext ext,
+               const int final_out) {
   Args a = args;
-  a.n = n;
-  a.splits = splits;
-  a.H = H;
-  a.Hkv = Hkv;
-  a.B = B;
+  Ext x = ext;
+  a.Hkv = (int)(heads_splits & 0xffff);
+  a.splits = (int)(heads_splits >> 16);
+  a.H = a.Hkv * G;
+  if (G == 1 && !(flags & KX_GQ1)) a.H = opaque(args.H);
   a.k = static_cast<const unsigned char *>(k);
   a.v = static_cast<const unsigned char *>(v);
   a.k_meta = static_cast<const __half2 *>(k_meta);
   a.v_meta = static_cast<const __half2 *>(v_meta);
-  a.q = static_cast<const float *>(q);
-  Ext x = ext;
-  x.nx = nx;
-  const int gy = G > 1 ? a.Hkv : a.H; // head groups per sequence
-  int split, hb, b;
-  if (x.nx > 0) { // fused step on a 1-D grid: a head group's splits share an XCD
-    const int m = a.B * gy / x.nx;
-    const int q = (int)(blockIdx.x / x.nx);
-    const int hg = (int)(blockIdx.x % x.nx) + x.nx * (q % m);
-    split = q / m;
-    b = hg / gy;
-    hb = hg % gy;
+  x.flags = flags;
+  x.seq_lens = static_cast<const int *>(n_chunk);
+  a.n = (int)(uint32_t)(uint64_t)n_chunk;
+  x.chunk = (int)((uint64_t)n_chunk >> 32);
+  if (!PAGED && (flags & KX_VARLEN)) a.n = opaque(args.n); // (row offsets; paged rows have none in n)
+  if constexpr (PAGED) {
+    a.block_table = static_cast<const int *>(q_or_table);
+    a.block_shift = (int)(flags >> KX_BS_SHIFT) & 15;
+    a.max_blocks = (int)(flags >> KX_MB_SHIFT);
+    if (a.max_blocks == (int)KX_MB_MAX) a.max_blocks = opaque(args.max_blocks);
   } else {
-    split = blockIdx.x;
-    hb = blockIdx.y;
-    b = blockIdx.z;
+    x.q = q_or_table;
+  }
+  const int nx = (int)(flags >> KX_NX_SHIFT) & 15;
+  int split = blockIdx.x, hb = blockIdx.y, b = blockIdx.z;
+  if (nx) {
+    split = blockIdx.z;
+    hb = blockIdx.x + nx * blockIdx.y;
+    b = 0;
+    if (flags & KX_HGDIV) {
+      const unsigned gy = G > 1 ? a.Hkv : a.H;
+      b = (unsigned)hb / gy;
+      hb -= b * gy;
+    }
   }
   decode_item<FMT, D, GQ, G, U, ORD, PAGED, WPB, false>(a, x, final_out, split, hb, b, nullptr);
 }
@@ -1117,7 +1220,7 @@ decode_partial(const int nx, const int n, const int splits, const int H, const i
 // does not pay.
 template <int FMT, int D, int GQ, int G, int U, int ORD, bool PAGED, int WPB>
 __global__ void __launch_bounds__(WPB * 64)
-decode_persistent(int, int, int, int, int, int, const void *, const void *, const void *, const void *,
+decode_persistent(uint32_t, uint32_t, const void *, const void *, const void *, const void *, const void *,
                   const void *, const Args a, const Ext x, const int final_out) {
   const int gy = G > 1 ? a.Hkv : a.H;
   __shared__ unsigned s_next;
@@ -1383,6 +1486,18 @@ inline hipError_t dev_info(DevInfo &out) {
   return hipSuccess;
 }
 
+// Tokens of a split with uniform lengths. The split kernel by itself
+// (partial_only) hands out its partials, and keeps the reference's chunks,
+// ceil(n / splits) tokens (runtime/kvf_kernels.cuh:147-150). A whole step
+// rounds them up to tiles: a chunk that starts or ends inside a tile shares
+// that tile with its neighbour, so a split reads up to one tile more than its
+// share, and every tile of a split that starts inside one is masked. Rounding
+// never adds a tile to the longest split.
+inline int uniform_chunk(int n, int splits, bool partial_only) {
+  const int per = (int)(((long long)n + splits - 1) / splits);
+  return partial_only ? per : (int)(((long long)per + TT - 1) / TT * TT);
+}
+
 template <int FMT, int D, int GQ, int G, int U, int ORD, bool PAGED>
 hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_t st) {
   const int gy = G > 1 ? a.Hkv : a.H;
@@ -1392,29 +1507,35 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   const bool fused = x.counters && !final_out && !l.partial_only;
   Ext xk = x;
   if (!fused) xk.counters = nullptr;
-  xk.nx = 0;
+  xk.q = x.q16 ? static_cast<const void *>(x.q16) : a.q;
+  xk.chunk = uniform_chunk(a.n, a.splits, l.partial_only);
+  uint32_t flags = (x.seq_lens ? KX_VARLEN : 0) | (x.q16 ? KX_Q16 : 0) | (a.H == a.Hkv ? KX_GQ1 : 0);
+  if (x.seq_lens && x.longest_first && a.B > 1 && a.B <= 64) flags |= KX_LPT;
+  if (PAGED)
+    flags |= (uint32_t)a.block_shift << KX_BS_SHIFT | std::min<uint32_t>(a.max_blocks, KX_MB_MAX) << KX_MB_SHIFT;
   if (fused) {
     // one launch: when the head groups divide evenly over the device's XCDs,
-    // a 1-D grid places every split of a head group on one XCD
+    // the XCD-affine grid places every split of a head group on one XCD
     DevInfo di;
     const hipError_t e = dev_info(di);
     if (e != hipSuccess) return e;
-    const int nhg = a.B * gy;
+    const long long nhg = (long long)a.B * gy;
     // (head-major rows only: with token-major rows every KV head sits at one
     // byte offset of each token's row, and one head per XCD made a paged
     // token-major batch of 8 sequences take 38 us fused against 28 us on the
     // (splits, heads, B) grid)
-    // (uniform lengths only: the 1-D order runs split by split over all head
+    // (uniform lengths only: the affine order runs split by split over all head
     // groups, which undoes longest-first and lets short sequences' splits
     // crowd out the long ones; a batch of 16 sequences with log-uniform
     // lengths up to 128k took 145 us fused on it against 94 us on the
     // (splits, heads, B) grid)
-    // (a 1-D grid holds at most 2^32 - 1 work-items: larger steps keep the
-    // 3-D grid)
-    if (ORD == ORD_HEAD && !x.seq_lens && di.nx > 1 && nhg % di.nx == 0 &&
+    // (a grid holds at most 2^32 - 1 work-items along it, and 65535
+    // workgroups in y: larger steps keep the plain grid)
+    if (ORD == ORD_HEAD && !x.seq_lens && di.nx > 1 && di.nx < 16 && nhg % di.nx == 0 && nhg / di.nx <= 65535 &&
         (long long)a.splits * nhg * block.x <= 0xffffffffLL) {
-      xk.nx = di.nx;
-      grid = dim3((unsigned)(a.splits * nhg));
+      flags |= (uint32_t)di.nx << KX_NX_SHIFT;
+      if (a.B > 1) flags |= KX_HGDIV;
+      grid = dim3((unsigned)di.nx, (unsigned)(nhg / di.nx), (unsigned)a.splits);
     }
   }
   const size_t lds = combine_lds<FMT, D, GQ, G>(a.warps);
@@ -1471,20 +1592,24 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
     if (queue) {
       kernel = pk;
       grid = dim3((unsigned)wgs);
-      xk.nx = 0;
     } else {
       xk.queue = nullptr;
     }
   }
   // the split kernel's leading scalars (see decode_partial; the persistent
-  // kernel takes the same list and reads Args)
-  const void *kp = a.k, *vp = a.v, *kmp = a.k_meta, *vmp = a.v_meta, *qp = a.q;
+  // kernel takes the same list and reads Args and Ext)
+  xk.flags = flags;
+  const uint32_t hs = (uint32_t)a.Hkv | (uint32_t)a.splits << 16;
+  const void *nc = x.seq_lens ? static_cast<const void *>(x.seq_lens)
+                              : reinterpret_cast<const void *>((uint64_t)(uint32_t)a.n |
+                                                               (uint64_t)(uint32_t)xk.chunk << 32);
+  const void *kp = a.k, *vp = a.v, *kmp = a.k_meta, *vmp = a.v_meta;
+  const void *qt = PAGED ? static_cast<const void *>(a.block_table) : xk.q;
   if (l.ev_start || l.ev_stop)
-    hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)lds, st, l.ev_start, l.ev_stop, 0, xk.nx, a.n, a.splits,
-                          a.H, a.Hkv, a.B, kp, vp, kmp, vmp, qp, a, xk, final_out);
+    hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)lds, st, l.ev_start, l.ev_stop, 0, flags, hs, nc, kp, vp,
+                          kmp, vmp, qt, a, xk, final_out);
   else
-    hipLaunchKernelGGL(kernel, grid, block, lds, st, xk.nx, a.n, a.splits, a.H, a.Hkv, a.B, kp, vp, kmp, vmp, qp,
-                       a, xk, final_out);
+    hipLaunchKernelGGL(kernel, grid, block, lds, st, flags, hs, nc, kp, vp, kmp, vmp, qt, a, xk, final_out);
   if (!final_out && !l.partial_only && !fused) return launch_merge_kernel<D>(a, x, st);
   return hipGetLastError();
 }

@@ -82,22 +82,21 @@ def _patches():
          # slot 7: where the wave runs (XCC_ID in the high word, HW_ID: CU, SIMD, wave slot)
          "  TS(7, ((unsigned long long)__builtin_amdgcn_s_getreg(0x1814) << 32) |\n"
          "        (unsigned)__builtin_amdgcn_s_getreg(0xF804));\n"),
-        ("kvf_kernels.hpp", "        compute(ring(Ui), k, mask_tag);\n        ++k;\n      });\n    }",
-         "        compute(ring(Ui), k, mask_tag);\n        if (k == 0) " + _stamp(1, "acc[0][0][0]") +
-         "\n        ++k;\n      });\n    }"),
-        ("kvf_kernels.hpp", "  // drain: the tiles still in flight, masked (a full tile computes the same)\n",
+        ("kvf_kernels.hpp", "      compute(ring(Ui), k + s);\n",
+         "      compute(ring(Ui), k + s);\n      if (k + s == 0) " + _stamp(1, "acc[0][0][0]") + "\n"),
+        ("kvf_kernels.hpp", "  // persistent step: thread 0 claims the workgroup's next item behind the\n",
          "  " + _stamp(2, "acc[0][0][0]") + "\n"
-         "  // drain: the tiles still in flight, masked (a full tile computes the same)\n"),
+         "  // persistent step: thread 0 claims the workgroup's next item behind the\n"),
         ("kvf_kernels.hpp", "  // ---- wave result: per head (m_run, l, m_true) and O[head][D] ---------------\n",
          "  " + _stamp(9, "acc[0][0][0]") + "\n"
          "  // ---- wave result: per head (m_run, l, m_true) and O[head][D] ---------------\n"),
-        ("kvf_kernels.hpp", "  // every LDS read of an output element is issued before any is used: the\n",
+        ("kvf_kernels.hpp", "  // A thread takes VPT neighbouring dims of one head, so the waves' weights\n",
          "  " + _stamp(3, "lane") + "\n"
-         "  // every LDS read of an output element is issued before any is used: the\n"),
+         "  // A thread takes VPT neighbouring dims of one head, so the waves' weights\n"),
         ("kvf_kernels.hpp",
          "    const int hq = G > 1 ? hkv * G + hh : hb;\n    const long long head = (long long)b * a.H + hq;\n",
          "    const int hq = G > 1 ? hkv * G + hh : hb;\n    const long long head = (long long)b * a.H + hq;\n"
-         "    if (idx0 + nthreads >= G * D) " + _stamp(10, "O") + "\n"),
+         "    " + _stamp(10, "O[0]") + "\n"),
         ("kvf_kernels.hpp",
          "    asm volatile(\"s_waitcnt vmcnt(0)\" ::: \"memory\");\n    __syncthreads();\n"
          "    if (threadIdx.x == 0)\n"

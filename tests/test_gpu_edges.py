@@ -1,0 +1,105 @@
+"""Decode steps at the sizes where the split kernel's paths part: waves with
+no, one, an odd and an even number of tiles; chunks and sequence ends inside a
+tile; the XCD-affine grid over several sequences; query heads that share a KV
+head without packing; a page table whose row is longer than the launch word
+holds. Each against the oracle's double-precision attention over the same
+dequantised cache.
+
+Tolerances. Every product enters as a binary16 hi/lo pair (22 bits) and sums
+are fp32: per head the steps measure up to 5e-6 (int8 with outlier channels),
+2e-6 (f16) and 3e-5 (int4:32, whose scales are 17 times larger). A pair whose
+halves do not belong together is off by a binary16 ulp of one element, 2^-11
+of its share of a score: 7e-5 to 6e-4 of a head. So heads are held to 2^-15
+(int8, f16), and int4 to 2^-13."""
+import numpy as np
+import pytest
+import torch
+
+import _oracle as O
+from _cases import Case, args, build, reference, run, vid
+from kvforge_amd import runtime as R
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    R.hip_lib()
+
+
+def worst_head(got, ref):
+    d = np.linalg.norm(got.astype(np.float64) - ref, axis=-1)
+    return float(np.max(d / np.maximum(np.linalg.norm(ref, axis=-1), 1e-30)))
+
+
+def limit(fmt):
+    return 2.0 ** -13 if fmt == R.FMT_INT4 else 2.0 ** -15
+
+
+@pytest.mark.parametrize("fmt,group", [(R.FMT_F16, 0), (R.FMT_INT8, 64), (R.FMT_INT8, 32)])
+@pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (16, 16, 64), (32, 4, 64)])
+def test_every_head_keeps_its_precision(fmt, group, H, Hkv, D):
+    b = build(Case(16, H, Hkv, D, 64, fmt, group, R.ORD_HEAD, 0, seed=3, outliers=True))
+    err = worst_head(run(b, 1), reference(b))
+    print(f"  {b.case.tag()}: worst head {err:.3g}", flush=True)
+    assert err < limit(fmt)
+
+
+@pytest.mark.parametrize("fmt,group,order,bt", [(R.FMT_F16, 0, R.ORD_HEAD, 0), (R.FMT_INT8, 64, R.ORD_HEAD, 16),
+                                                (R.FMT_INT8, 64, R.ORD_TOKEN, 0), (R.FMT_INT4, 32, R.ORD_TOKEN, 16)])
+def test_tiles_of_a_wave(fmt, group, order, bt):
+    for n in (1, 31, 33, 127, 128, 160, 257, 385, 641, 1003):
+        b = build(Case(1, 8, 2, 128, n, fmt, group, order, bt, seed=n))
+        for splits, warps, unroll in ((1, 4, 2), (1, 8, 4), (3, 4, 2), (8, 4, 4), (16, 8, 2)):
+            print(f"  {b.case.tag()} S{splits} w{warps} u{unroll}", flush=True)
+            assert worst_head(run(b, splits, unroll=unroll, warps=warps), reference(b)) < limit(fmt)
+
+
+@pytest.mark.parametrize("B,H,Hkv", [(1, 32, 8), (4, 8, 2), (3, 64, 16), (2, 16, 16)])
+def test_one_launch_over_the_affine_grid(B, H, Hkv):
+    b = build(Case(B, H, Hkv, 128, 500, R.FMT_INT8, 64, R.ORD_HEAD, 0, seed=B))
+    counters = R.fused_counters(B, Hkv)
+    for splits in (2, 5):
+        b.out.fill_(float("nan"))
+        R.launch_fused(vid(b, True, 2), args(b, splits), counters)
+        torch.cuda.synchronize()
+        assert worst_head(b.out.cpu().numpy(), reference(b)) < limit(R.FMT_INT8)
+        assert not bool(counters.any())
+
+
+@pytest.mark.parametrize("bt", [0, 16])
+def test_unpacked_query_heads(bt):
+    b = build(Case(2, 12, 3, 64, 300, R.FMT_INT8, 32, R.ORD_TOKEN, bt, seed=7))
+    assert worst_head(run(b, 4, pack=False), reference(b)) < limit(R.FMT_INT8)
+
+
+@pytest.mark.parametrize("max_blocks", [(1 << 19) - 2, (1 << 19) - 1, (1 << 19) + 3])
+def test_long_page_table_rows(max_blocks):
+    b = build(Case(2, 8, 2, 128, 200, R.FMT_INT8, 64, R.ORD_HEAD, 16, seed=9))
+    table = torch.zeros((2, max_blocks), dtype=torch.int32, device="cuda:0")
+    table[:, :b.max_blocks] = b.table.view(2, b.max_blocks)
+    b.table, b.max_blocks = table, max_blocks
+    assert worst_head(run(b, 2), reference(b)) < limit(R.FMT_INT8)
+
+
+@pytest.mark.parametrize("fmt,group,order", [(R.FMT_F16, 0, R.ORD_TOKEN), (R.FMT_INT8, 64, R.ORD_HEAD),
+                                             (R.FMT_INT4, 32, R.ORD_TOKEN)])
+@pytest.mark.parametrize("bt", [0, 16])
+def test_unequal_lengths(fmt, group, order, bt):
+    b = build(Case(5, 8, 2, 128, 300, fmt, group, order, bt, seed=11))
+    lens = np.array([300, 0, 1, 33, 160], np.int32)
+    ref = np.zeros((5, 8, 128))
+    for i, n in enumerate(lens):
+        if n:
+            ref[i] = O.reference_attention(b.q_host[i:i + 1], np.ascontiguousarray(b.kdeq[i:i + 1, :, :n]),
+                                           np.ascontiguousarray(b.vdeq[i:i + 1, :, :n]))[0]
+    lens_d = torch.from_numpy(lens).cuda()
+    for splits, flags in ((1, 0), (4, 0), (4, R.VARLEN_LONGEST_FIRST)):
+        b.out.fill_(float("nan"))
+        R.launch_varlen(vid(b, True, 2), args(b, splits), lens_d, flags=flags)
+        torch.cuda.synchronize()
+        got = b.out.cpu().numpy()
+        assert not got[1].any()
+        assert worst_head(got, ref) < limit(fmt)
