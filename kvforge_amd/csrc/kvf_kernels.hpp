@@ -1258,7 +1258,13 @@ decode_persistent(uint32_t, uint32_t, const void *, const void *, const void *, 
 // because it runs once per head group from a cold instruction cache. Empty
 // splits (max -inf) and slots past the split count weigh nothing (every
 // split writes its row on every call, an empty one zeros, so every row read
-// is finite); more than 32 splits fold with a running max. Loads are
+// is finite); more than 32 splits fold with a running max. A chunk costs its
+// loads and sums whether its splits are there or not, in the one workgroup that
+// everything waits for, so octets past the last split are left out (one-launch
+// steps on MI355X: 1003 tokens in 8 splits 7.0 -> 6.4 us, a paged batch of 8
+// sequences in 8 splits 26.4 -> 25.1 us, 2048 tokens in 16 splits 7.1 -> 6.8 us;
+// in the stand-alone merge, one workgroup a head, the same gained nothing).
+// Loads are
 // device-coherent raw buffer loads through descriptors over the head's rows
 // (a split past the end reads zero).
 //
@@ -1272,6 +1278,7 @@ template <int D, int G, int NW>
 __device__ __forceinline__ void merge_heads(const Args &a, const Ext &x, long long head0, bool dry) {
   constexpr int EL = D / 64; // output dims per lane
   constexpr int MCH = 32;    // splits per round trip
+  constexpr int OCT = 8;     // of which a group past the last split is left out
   constexpr int CPOL = CPOL_SC1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1287,8 +1294,13 @@ __device__ __forceinline__ void merge_heads(const Args &a, const Ext &x, long lo
       const int sl = s0 + (lane & (MCH - 1));
       const i32x2_t p = __builtin_amdgcn_raw_buffer_load_b64(rml, sl * 8, 0, CPOL);
       Raw<EL * 4> o[MCH];
+      static_for<MCH / OCT>([&](auto Q) __attribute__((always_inline)) {
+        constexpr int q = OCT * decltype(Q)::value;
+        if (q == 0 || s0 + q < S) {
 #pragma unroll
-      for (int i = 0; i < MCH; ++i) bload<EL * 4, CPOL>(ro, ((s0 + i) * D + lane * EL) * 4, o[i]);
+          for (int i = q; i < q + OCT; ++i) bload<EL * 4, CPOL>(ro, ((s0 + i) * D + lane * EL) * 4, o[i]);
+        }
+      });
       // every load of the chunk goes out before any is used: one round trip
       __builtin_amdgcn_sched_barrier(0);
       // (elements go through plain ints: clang's __builtin_bit_cast of an
@@ -1320,12 +1332,17 @@ __device__ __forceinline__ void merge_heads(const Args &a, const Ext &x, long lo
       L = fmaf(L, alpha, lw);
 #pragma unroll
       for (int e = 0; e < EL; ++e) O[e] *= alpha;
+      static_for<MCH / OCT>([&](auto Q) __attribute__((always_inline)) {
+        constexpr int q = OCT * decltype(Q)::value;
+        if (q == 0 || s0 + q < S) {
 #pragma unroll
-      for (int i = 0; i < MCH; ++i) {
-        const float wi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), i));
+          for (int i = q; i < q + OCT; ++i) {
+            const float wi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), i));
 #pragma unroll
-        for (int e = 0; e < EL; ++e) O[e] = fmaf(__builtin_bit_cast(float, o[i].w[e]), wi, O[e]);
-      }
+            for (int e = 0; e < EL; ++e) O[e] = fmaf(__builtin_bit_cast(float, o[i].w[e]), wi, O[e]);
+          }
+        }
+      });
       M = Mc;
     }
     if (dry) {
