@@ -83,8 +83,9 @@ __device__ __forceinline__ uint32_t code_div(float a, float sc, float levels) {
 
 // Quantizes a row's 8 elements [8c, 8c + 8) and writes them, and the group's
 // (scale, zero) from its first lane, to physical row `prow`. All lanes of a
-// row call it together (the reductions stay inside a row).
-template <int FMT, int D, int GQ>
+// row call it together (the reductions stay inside a row). NT: the codes pass
+// the caches by (a whole prompt's rows), or stay for the step that reads them.
+template <int FMT, int D, int GQ, bool NT>
 __device__ __forceinline__ void put_row(f4u v0, f4u v1, int c, long long prow, unsigned char *data, uint32_t *meta) {
   constexpr int ROW = D * bits_of<FMT>() / 8;
   float e[8];
@@ -96,7 +97,8 @@ __device__ __forceinline__ void put_row(f4u v0, f4u v1, int c, long long prow, u
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       w[k] = __builtin_bit_cast(uint32_t, (half2_t){(_Float16)e[2 * k], (_Float16)e[2 * k + 1]});
-    *reinterpret_cast<u4u *>(to) = w;
+    if constexpr (NT) __builtin_nontemporal_store(w, reinterpret_cast<u4u *>(to));
+    else *reinterpret_cast<u4u *>(to) = w;
   } else {
     constexpr float LEVELS = FMT == FMT_INT8 ? 255.f : 15.f;
     constexpr int LPG = GQ / 8; // lanes per group
@@ -133,92 +135,76 @@ __device__ __forceinline__ void put_row(f4u v0, f4u v1, int c, long long prow, u
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         w[k] = q[4 * k] | q[4 * k + 1] << 8 | q[4 * k + 2] << 16 | q[4 * k + 3] << 24;
-      *reinterpret_cast<u2u *>(to) = w;
+      if constexpr (NT) __builtin_nontemporal_store(w, reinterpret_cast<u2u *>(to));
+      else *reinterpret_cast<u2u *>(to) = w;
     } else {
       uint32_t w = 0;
 #pragma unroll
       for (int k = 0; k < 8; ++k) w |= q[k] << (4 * k); // even elements in the low nibble
-      *reinterpret_cast<u1u *>(to) = w;
+      if constexpr (NT) __builtin_nontemporal_store(w, reinterpret_cast<u1u *>(to));
+      else *reinterpret_cast<u1u *>(to) = w;
     }
   }
 }
 
-// A wave takes R * 512 / D neighbouring work items; all their loads go out
-// before the first is used. The items' (sequence, head, token) come from one
-// scalar division per load of a wave, its first item's, and a carry per lane
-// (per-lane divisions were as many cycles as the quantizing).
+// A wave takes 512 / D neighbouring work items, a load of 16 bytes twice a
+// lane. Items' (sequence, head, token) come from one scalar division per wave,
+// its first item's, and a carry per lane (per-lane divisions were as many
+// cycles as the quantizing). More items a wave, 2, 4 or 8 loads in flight a
+// lane, were each slower than more waves (2: 64.8, 4: 68.2, 8: 76.5 us where 1
+// takes 62.3); the codes' stores are nontemporal, the rows' loads are not (they
+// are often still cached: with nontemporal loads 8000 tokens 16.8 -> 18.5 us).
 // Measured on MI355X, K and V of one layer with 8 KV heads of 128: 32768
-// tokens in int8:64, head-major contiguous, 339 -> 68 us (5.0 TB/s read and
-// written, a large copy's 5.2); 4 x 4093 tokens in int4:32, paged token-major,
-// 180 -> 36 us (4.3 TB/s). Before, a wave took one row, a lane single elements
-// with byte stores, and every element one division.
-template <int FMT, int D, int GQ, int R>
+// tokens in int8:64, head-major contiguous, 339 -> 62 us (5.5 TB/s read and
+// written; a large copy reaches 5.2); 4 x 4093 tokens in int4:32, paged
+// token-major, 180 -> 35 us (4.4 TB/s). Before, a wave took one row, a lane
+// single elements with byte stores, and every element one division.
+template <int FMT, int D, int GQ>
 __global__ void __launch_bounds__(256)
 quantize_place_kernel(const float *__restrict__ x, unsigned char *__restrict__ data, uint32_t *__restrict__ meta,
                       const Place p) {
-  constexpr int LPR = D / 8;         // lanes per row
-  constexpr int RPW = 64 / LPR;      // rows per wave and load
+  constexpr int LPR = D / 8;    // lanes per row
+  constexpr int RPW = 64 / LPR; // rows per wave
   const int lane = threadIdx.x & 63;
-  const uint32_t wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c = lane % LPR;          // the lane's elements are [8c, 8c + 8)
-  bool ok[R];
-  uint32_t b[R], h[R], t[R], item[R];
-  int page[R];
-  f4u v[R][2];
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    const uint32_t i0 = (wave * R + j) * RPW, o = lane / LPR;
-    ok[j] = i0 + o < p.rows;
-    // past the end: the last row again, loaded and not stored
-    const uint32_t i = item[j] = ok[j] ? i0 + o : p.rows - 1;
-    uint32_t in, mid;
-    if (p.inner.div >= RPW && i0 + RPW <= p.rows) {
-      const uint32_t rest0 = p.inner.quot(i0), b0 = p.outer.quot(rest0);
-      in = i0 - rest0 * p.inner.div + o;
-      mid = rest0 - b0 * p.outer.div;
-      b[j] = b0;
-      if (in >= p.inner.div) {
-        in -= p.inner.div;
-        ++mid;
-      }
-      if (mid >= p.outer.div) {
-        mid = 0;
-        ++b[j];
-      }
-    } else {
-      const uint32_t rest = p.inner.quot(i);
-      in = i - rest * p.inner.div;
-      b[j] = p.outer.quot(rest);
-      mid = rest - b[j] * p.outer.div;
+  const int c = lane % LPR;     // the lane's elements are [8c, 8c + 8)
+  const uint32_t i0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RPW, o = lane / LPR;
+  const bool ok = i0 + o < p.rows;
+  // past the end: the last row again, loaded and not stored
+  const uint32_t item = ok ? i0 + o : p.rows - 1;
+  uint32_t in, mid, b;
+  if (p.inner.div >= RPW && i0 + RPW <= p.rows) {
+    const uint32_t rest0 = p.inner.quot(i0), b0 = p.outer.quot(rest0);
+    in = i0 - rest0 * p.inner.div + o;
+    mid = rest0 - b0 * p.outer.div;
+    b = b0;
+    if (in >= p.inner.div) {
+      in -= p.inner.div;
+      ++mid;
     }
-    h[j] = p.order == ORD_HEAD ? mid : in;
-    t[j] = p.order == ORD_HEAD ? in : mid;
+    if (mid >= p.outer.div) {
+      mid = 0;
+      ++b;
+    }
+  } else {
+    const uint32_t rest = p.inner.quot(item);
+    in = item - rest * p.inner.div;
+    b = p.outer.quot(rest);
+    mid = rest - b * p.outer.div;
   }
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    // logical row (b Hkv + h) n + t; head-major items are in that order already
-    const uint32_t src = p.order == ORD_HEAD ? item[j] : (b[j] * p.Hkv + h[j]) * p.n + t[j];
-    const float *xr = x + (long long)src * D + c * 8;
-    v[j][0] = *reinterpret_cast<const f4u *>(xr);
-    v[j][1] = *reinterpret_cast<const f4u *>(xr + 4);
-  }
+  const uint32_t h = p.order == ORD_HEAD ? mid : in;
+  const uint32_t t = p.order == ORD_HEAD ? in : mid;
+  // logical row (b Hkv + h) n + t; head-major items are in that order already
+  const uint32_t src = p.order == ORD_HEAD ? item : (b * p.Hkv + h) * p.n + t;
+  const float *xr = x + (long long)src * D + c * 8;
+  const f4u v0 = *reinterpret_cast<const f4u *>(xr), v1 = *reinterpret_cast<const f4u *>(xr + 4);
+  long long prow = item; // the physical row; contiguous: the item itself
   if (p.bt) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) page[j] = p.table[(long long)b[j] * p.max_blocks + p.page.quot(t[j])];
+    const uint32_t blk = p.page.quot(t), off = t - blk * p.bt;
+    prow = (long long)p.table[(long long)b * p.max_blocks + blk] * (p.Hkv * p.bt) +
+           (p.order == ORD_HEAD ? h * p.bt + off : off * p.Hkv + h);
   }
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    // a row's lanes leave together (the group reductions stay inside a row)
-    if (!ok[j]) continue;
-    long long prow; // the physical row
-    if (p.bt) {
-      const uint32_t in = t[j] - p.page.quot(t[j]) * p.bt;
-      prow = (long long)page[j] * (p.Hkv * p.bt) + (p.order == ORD_HEAD ? h[j] * p.bt + in : in * p.Hkv + h[j]);
-    } else {
-      prow = item[j];
-    }
-    put_row<FMT, D, GQ>(v[j][0], v[j][1], c, prow, data, meta);
-  }
+  // (a row's lanes go together: the group reductions stay inside a row)
+  if (ok) put_row<FMT, D, GQ, true>(v0, v1, c, prow, data, meta);
 }
 
 // One token per sequence: a workgroup is one wave on 64 * 8 / D neighbouring
@@ -262,7 +248,7 @@ append_kernel(const float *__restrict__ x, const int *__restrict__ positions, co
     } else {
       prow = head_major ? ((long long)b * Hkv + h) * limit + t : ((long long)b * limit + t) * Hkv + h;
     }
-    if (ok && h < Hkv) put_row<FMT, D, GQ>(v0, v1, c, prow, data, meta);
+    if (ok && h < Hkv) put_row<FMT, D, GQ, false>(v0, v1, c, prow, data, meta);
     b += 65535;
   } while (b < B);
 }
@@ -302,15 +288,8 @@ template <int FMT, int D, int GQ> hipError_t launch_quantize(const Call &q, hipS
   p.outer = FastDiv(q.order == ORD_HEAD ? q.Hkv : q.n);
   p.page = FastDiv(q.bt ? q.bt : 1);
   p.table = q.table;
-  // 4 loads a lane in flight where the rows give every SIMD of the chip two
-  // waves of them; fewer rows spread over more waves
-  if (p.rows >= 2048u * 4 * RPW) {
-    const dim3 grid((p.rows + 16 * RPW - 1) / (16 * RPW));
-    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 4>), grid, dim3(256), 0, st, q.x, q.data, q.meta, p);
-  } else {
-    const dim3 grid((p.rows + 4 * RPW - 1) / (4 * RPW));
-    hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ, 1>), grid, dim3(256), 0, st, q.x, q.data, q.meta, p);
-  }
+  const dim3 grid((p.rows + 4 * RPW - 1) / (4 * RPW));
+  hipLaunchKernelGGL((quantize_place_kernel<FMT, D, GQ>), grid, dim3(256), 0, st, q.x, q.data, q.meta, p);
   return hipGetLastError();
 }
 
