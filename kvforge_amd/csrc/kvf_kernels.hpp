@@ -1141,8 +1141,8 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
 }
 
 // The split kernel: a workgroup runs the one item its grid position names:
-// (split, head group, sequence) = blockIdx on the plain grid. On the fused
-// step's XCD-affine grid (nx, head groups / nx, splits), nx the device's XCDs,
+// (split, head group, sequence) = blockIdx on the plain grid. On the
+// XCD-affine grid (nx, head groups / nx, splits), nx the device's XCDs,
 // it is split z of head group x + nx * y: under the round-robin dispatch of
 // workgroups to XCDs every split of a head group runs on one XCD (the merge is
 // correct wherever they run: it publishes through the device-coherent level).
@@ -1530,9 +1530,16 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   if (x.seq_lens && x.longest_first && a.B > 1 && a.B <= 64) flags |= KX_LPT;
   if (PAGED)
     flags |= (uint32_t)a.block_shift << KX_BS_SHIFT | std::min<uint32_t>(a.max_blocks, KX_MB_MAX) << KX_MB_SHIFT;
-  if (fused) {
-    // one launch: when the head groups divide evenly over the device's XCDs,
-    // the XCD-affine grid places every split of a head group on one XCD
+  // XCD-affine grid: when the head groups divide evenly over the device's XCDs,
+  // every split of a head group on one XCD. The one-launch step merges there.
+  // In two launches it pays by the stream alone, an XCD then reading a few long
+  // runs of rows instead of a piece of every head's: GQA 32/8 32k int8:64 (67 MB
+  // of rows) 16.7-17.1 -> 16.2-16.3 us, a paged f16 batch of 4 (75 MB) 17.2 ->
+  // 16.6, MHA 4k f16 (67 MB) 15.0 -> 14.8. Below about 1.5 times the L2s' 32 MB
+  // it does not (1 MB 6.85 -> 6.90, 4 MB 6.94 -> 7.03, int4 d64 of 34 MB 16.7 ->
+  // 16.9; 38 MB of int8 12.2 -> 12.0), so those keep the plain grid.
+  const double payload = 2.0 * a.B * a.Hkv * (double)a.n * Geo<FMT, D, GQ, G>::ROW;
+  if (fused || (!final_out && !l.partial_only && !x.queue && payload >= 48.0 * (1 << 20))) {
     DevInfo di;
     const hipError_t e = dev_info(di);
     if (e != hipSuccess) return e;

@@ -103,3 +103,21 @@ def test_unequal_lengths(fmt, group, order, bt):
         got = b.out.cpu().numpy()
         assert not got[1].any()
         assert worst_head(got, ref) < limit(fmt)
+
+
+@pytest.mark.parametrize("B,Hkv,n", [(1, 8, 24575), (1, 8, 24576), (2, 4, 24601), (1, 3, 65536)])
+def test_large_two_launch_steps_on_either_grid(B, Hkv, n):
+    # 48 MiB of rows from n = 24576 on (8 head groups; 3 do not divide over the
+    # XCDs): the step against the partial kernel and the merge by themselves,
+    # which run on the plain grid and the reference's chunks. Only fp32 sums
+    # differ: 1e-5.
+    b = build(Case(B, 4 * Hkv, Hkv, 128, n, R.FMT_INT8, 64, R.ORD_HEAD, 0, seed=n), check_cache=False)
+    a = args(b, 12)
+    R.launch(vid(b, True, 2), a)
+    torch.cuda.synchronize()
+    got = b.out.cpu().numpy().copy()
+    b.out.fill_(float("nan"))
+    R.launch_partial(vid(b, True, 2), a)
+    R.launch_merge(128, a)
+    torch.cuda.synchronize()
+    assert worst_head(got, b.out.cpu().numpy().astype(np.float64)) < 1e-5
