@@ -46,7 +46,7 @@ struct Ext {
   // lengths)
   const void *q = nullptr;
   uint32_t flags = 0;
-  int chunk = 0;
+  uint32_t chunk = 0;
 };
 
 // How a decode step is enqueued: the split kernel alone (partial_only), and

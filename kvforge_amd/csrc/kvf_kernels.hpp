@@ -67,6 +67,7 @@
 #include "kvf_abi.h"
 #include "kvf_ext.hpp"
 #include "kvf_registry.h"
+#include "kvf_split.hpp"
 
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
@@ -87,8 +88,7 @@ typedef int32_t i32x2_t __attribute__((ext_vector_type(2)));
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int SUB = 16;                  // tokens per sub-tile (MFMA rows)
-constexpr int TT = 32;                   // tokens per tile (PV MFMA k)
+constexpr int SUB = 16;                  // tokens per sub-tile (MFMA rows); a tile is TT = 32 (kvf_split.hpp)
 constexpr float TAU = 8.0f;              // rescale threshold, log2 units
 constexpr float CODE_SHIFT = 16384.f;    // 2^14: code * 2^-24 (subnormal) -> code * 2^-10
 constexpr float CODE_UNIT = 1024.f;      // 2^10: undoes the codes' scale in the MFMAs
@@ -432,7 +432,7 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   if (G == 1 && !(x.flags & KX_GQ1)) hkv = hb / (a.H / a.Hkv);
 
   // The split's tiles: with uniform lengths a contiguous chunk of Ext::chunk
-  // tokens, [t0, t1) (see uniform_chunk). With per-sequence lengths:
+  // tokens, [t0, t1) (see launch_group). With per-sequence lengths:
   // - paged: every S-th tile, tiles split, split + S, ... below the
   //   sequence's length, so the tiles and their page ids are known before the
   //   length arrives;
@@ -497,13 +497,14 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   }
   if (strided) {
     t1 = len;
-    const int tt = (len + TT - 1) / TT;
+    const int tt = tiles_of(len);
     n_tiles = tt > split ? (int)((unsigned)(tt - split + a.splits - 1) / (unsigned)a.splits) : 0;
   } else {
-    int chunk = x.chunk;
-    if (varlen) chunk = ((int)((unsigned)(len + a.splits - 1) / (unsigned)a.splits) + TT - 1) / TT * TT;
-    t0 = split * chunk;
-    t1 = min(len, t0 + chunk);
+    uint32_t chunk = x.chunk;
+    if (varlen) chunk = split_chunk(len, a.splits, true);
+    const TokenRange range = split_range(len, chunk, split);
+    t0 = range.t0;
+    t1 = range.t1;
     tile0 = t0 / TT;
     n_tiles = t1 > t0 ? (t1 - 1) / TT - tile0 + 1 : 0;
   }
@@ -578,7 +579,7 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   // d128 head-major 28.7 -> 27.3 us.
   // Descriptors cover the tokens' strides: a token-major one ends up to a
   // stride past the last row, where no lane's offset points.
-  const int range_end = strided ? len : min(len, (tile0 + n_tiles) * TT);
+  const int range_end = strided ? len : (int)min((uint32_t)len, (uint32_t)(tile0 + n_tiles) * TT);
   int tnext = (tile0 + tstep * wave) * TT;          // first token of the next tile
   int knext = 0;
   int left = nk > 0 ? max(range_end - tnext, 0) : 0;
@@ -827,11 +828,11 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
     // in. Wave-uniform, a branch inside the one body that every tile runs: a
     // body of its own for such tiles made the kernel half as large again and
     // cost copies of the first tile's registers where the two met.
-    if (tbase < t0 || tbase + TT > t1) {
+    if (tbase < t0 || t1 - tbase < TT) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int t = tbase + tau(r, i);
-        const bool ok = t >= t0 && t < t1;
+        const uint32_t t = (uint32_t)tbase + tau(r, i); // (the last tile may end past 2^31)
+        const bool ok = t >= (uint32_t)t0 && t < (uint32_t)t1;
         s[i] = ok ? s[i] : -INFINITY;
 #pragma unroll
         for (int w = 0; w < VW; ++w) buf.v[i].w[w] = ok ? buf.v[i].w[w] : 0u;
@@ -843,8 +844,8 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       if constexpr (QMETA) {
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
-          const int t = tbase + st * SUB + 4 * r + (c & 3); // the lane's word
-          const bool ok = t >= t0 && t < t1;
+          const uint32_t t = (uint32_t)tbase + st * SUB + 4 * r + (c & 3); // the lane's word
+          const bool ok = t >= (uint32_t)t0 && t < (uint32_t)t1;
 #pragma unroll
           for (int p = 0; p < PASSES; ++p) buf.vmr[st].w[p] = ok ? buf.vmr[st].w[p] : 0u;
         }
@@ -1180,7 +1181,7 @@ decode_partial(const uint32_t flags, const uint32_t heads_splits, const void *n_
   x.flags = flags;
   x.seq_lens = static_cast<const int *>(n_chunk);
   a.n = (int)(uint32_t)(uint64_t)n_chunk;
-  x.chunk = (int)((uint64_t)n_chunk >> 32);
+  x.chunk = (uint32_t)((uint64_t)n_chunk >> 32);
   if (!PAGED && (flags & KX_VARLEN)) a.n = opaque(args.n); // (row offsets; paged rows have none in n)
   if constexpr (PAGED) {
     a.block_table = static_cast<const int *>(q_or_table);
@@ -1503,18 +1504,6 @@ inline hipError_t dev_info(DevInfo &out) {
   return hipSuccess;
 }
 
-// Tokens of a split with uniform lengths. The split kernel by itself
-// (partial_only) hands out its partials, and keeps the reference's chunks,
-// ceil(n / splits) tokens (runtime/kvf_kernels.cuh:147-150). A whole step
-// rounds them up to tiles: a chunk that starts or ends inside a tile shares
-// that tile with its neighbour, so a split reads up to one tile more than its
-// share, and every tile of a split that starts inside one is masked. Rounding
-// never adds a tile to the longest split.
-inline int uniform_chunk(int n, int splits, bool partial_only) {
-  const int per = (int)(((long long)n + splits - 1) / splits);
-  return partial_only ? per : (int)(((long long)per + TT - 1) / TT * TT);
-}
-
 template <int FMT, int D, int GQ, int G, int U, int ORD, bool PAGED>
 hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_t st) {
   const int gy = G > 1 ? a.Hkv : a.H;
@@ -1525,7 +1514,13 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   Ext xk = x;
   if (!fused) xk.counters = nullptr;
   xk.q = x.q16 ? static_cast<const void *>(x.q16) : a.q;
-  xk.chunk = uniform_chunk(a.n, a.splits, l.partial_only);
+  // Uniform lengths: the split kernel by itself (partial_only) hands out its
+  // partials, and keeps the reference's chunks. A whole step's are whole tiles:
+  // a chunk that starts or ends inside a tile shares that tile with its
+  // neighbour, so a split reads up to one tile more than its share, and every
+  // tile of a split that starts inside one is masked. Rounding never adds a
+  // tile to the longest split.
+  xk.chunk = split_chunk(a.n, a.splits, !l.partial_only);
   uint32_t flags = (x.seq_lens ? KX_VARLEN : 0) | (x.q16 ? KX_Q16 : 0) | (a.H == a.Hkv ? KX_GQ1 : 0);
   if (x.seq_lens && x.longest_first && a.B > 1 && a.B <= 64) flags |= KX_LPT;
   if (PAGED)
@@ -1626,7 +1621,7 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   const uint32_t hs = (uint32_t)a.Hkv | (uint32_t)a.splits << 16;
   const void *nc = x.seq_lens ? static_cast<const void *>(x.seq_lens)
                               : reinterpret_cast<const void *>((uint64_t)(uint32_t)a.n |
-                                                               (uint64_t)(uint32_t)xk.chunk << 32);
+                                                               (uint64_t)xk.chunk << 32);
   const void *kp = a.k, *vp = a.v, *kmp = a.k_meta, *vmp = a.v_meta;
   const void *qt = PAGED ? static_cast<const void *>(a.block_table) : xk.q;
   if (l.ev_start || l.ev_stop)

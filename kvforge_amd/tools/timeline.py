@@ -147,6 +147,7 @@ def build(vid, inst):
         if files[f].count(old) != 1:
             raise SystemExit(f"timeline: the stamp anchor in {f} is gone: {old[:60]!r}")
         files[f] = files[f].replace(old, new)
+    files["kvf_split.hpp"] = open(os.path.join(src, "kvf_split.hpp")).read()
     for f, text in files.items():
         with open(os.path.join(csrc, f), "w") as fh:
             fh.write(text)
