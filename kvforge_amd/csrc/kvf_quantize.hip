@@ -317,8 +317,14 @@ hipError_t quantize_rows(const Call &q, int d, hipStream_t st) {
   if (q.fmt != FMT_F16) {
     if (!q.meta || (q.group != 32 && q.group != 64 && q.group != 128) || q.group > d) return hipErrorInvalidValue;
   }
-  // work items are 31-bit (a kernel of one row per 64 threads ended at 2^26 rows)
-  if ((long long)q.B * q.Hkv * (q.positions ? 1 : q.n) > 0x7fffffffLL) return hipErrorInvalidValue;
+  // A grid dimension holds 2^32 - 1 work-items, and a row takes d / 8 of x: all
+  // rows of a bulk call, one sequence's of an append, in whole workgroups (256
+  // and 64 threads). That is 2^28 (d 128) and 2^29 rows (d 64), and row numbers
+  // fit 31 bits below it.
+  const int per_group = (q.positions ? 64 : 256) / (d / 8);
+  const long long most = 0xffffffffLL / (d / 8) / per_group * per_group;
+  const long long heads = q.positions ? q.Hkv : (long long)q.B * q.Hkv;
+  if (heads > most || (!q.positions && heads * q.n > most)) return hipErrorInvalidValue;
   return d == 64 ? launch_format<64>(q, st) : launch_format<128>(q, st);
 }
 

@@ -149,3 +149,19 @@ def test_noalloc_entry_rejects_steps_beyond_its_scratch():
                                                 None) == R.HIP_ERROR_NOT_FOUND
     text = open(os.path.join(INCLUDE, "kvf_abi.h")).read()
     assert "#define KVF_SCRATCH_BYTES (16u << 20)" in text
+
+
+@pytest.mark.skipif(not os.path.exists(R.HIP_LIB), reason="libkvf_hip.so not built")
+def test_quantize_refuses_more_rows_than_a_grid_holds():
+    # a grid dimension holds 2^32 - 1 work-items, and a row takes d / 8 of them
+    # in whole workgroups; an append's limit is on one sequence's heads. Refused
+    # before any device call (the pointers are never followed)
+    lib = R.hip_lib()
+    p = ctypes.c_void_p(4096)
+    for d, most in ((128, 2 ** 28 - 16), (64, 2 ** 29 - 32)):
+        for B, Hkv, n in ((1, 1, most + 1), (1, most + 1, 1), (most // 8 + 1, 4, 2), (2 ** 31 - 1, 2 ** 31 - 1, 2 ** 31 - 1)):
+            assert lib.kvf_quantize_place(R.FMT_INT8, 64, d, p, B, Hkv, n, R.ORD_HEAD, 0, None, 0, p, p,
+                                          None) == R.HIP_ERROR_INVALID_VALUE, (d, B, Hkv, n)
+        for B, Hkv in ((1, most + 32), (7, 2 ** 31 - 1)):
+            assert lib.kvf_append_tokens(R.FMT_INT8, 64, d, p, B, Hkv, 5, p, R.ORD_TOKEN, 0, None, 0, p, p,
+                                         None) == R.HIP_ERROR_INVALID_VALUE, (d, B, Hkv)
