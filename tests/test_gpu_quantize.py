@@ -1,4 +1,4 @@
-"""The GPU quantize/place kernel byte for byte against a float32 restatement
+"""The GPU quantize/place and append kernels byte for byte against a float32 restatement
 of the reference's quantizer (runtime/kvf_host.h:72-121): the correctly
 rounded quotient (x - zero) / scale rounded half away from zero, over rows
 that sit on and beside rounding ties, scales that leave binary16, infinities
@@ -92,11 +92,13 @@ SHAPES = [  # B, Hkv, n, bt
 ]
 
 
+FORMATS = [(R.FMT_F16, 0, 64), (R.FMT_F16, 0, 128), (R.FMT_INT8, 32, 64), (R.FMT_INT8, 64, 64), (R.FMT_INT8, 32, 128),
+           (R.FMT_INT8, 64, 128), (R.FMT_INT8, 128, 128), (R.FMT_INT4, 32, 64), (R.FMT_INT4, 64, 64),
+           (R.FMT_INT4, 32, 128), (R.FMT_INT4, 64, 128), (R.FMT_INT4, 128, 128)]
+
+
 @pytest.mark.parametrize("order", [R.ORD_HEAD, R.ORD_TOKEN], ids=["hm", "tm"])
-@pytest.mark.parametrize("fmt,group,d", [(R.FMT_F16, 0, 64), (R.FMT_F16, 0, 128), (R.FMT_INT8, 32, 64),
-                                         (R.FMT_INT8, 64, 64), (R.FMT_INT8, 32, 128), (R.FMT_INT8, 64, 128),
-                                         (R.FMT_INT8, 128, 128), (R.FMT_INT4, 32, 64), (R.FMT_INT4, 64, 64),
-                                         (R.FMT_INT4, 32, 128), (R.FMT_INT4, 64, 128), (R.FMT_INT4, 128, 128)])
+@pytest.mark.parametrize("fmt,group,d", FORMATS)
 def test_quantized_bytes(fmt, group, d, order):
     for B, Hkv, n, bt in SHAPES:
         for off in (0, 1):  # buffers at a 256-byte boundary, and one element past it
@@ -122,3 +124,67 @@ def test_quantized_bytes(fmt, group, d, order):
                 assert np.array_equal(md.cpu().numpy().view(np.uint32), wmeta.reshape(-1))
             for raw in keep[1:]:  # nothing beyond the buffers
                 assert bool((raw[-64:] == 0xA5).all())
+
+
+def appended(fmt, group, d, B, Hkv, n, order, bt, off, positions, seed):
+    """One append call of a row per (sequence, head) into buffers filled with
+    0xA5: the rows at the positions inside the layout hold their codes and
+    words, and nothing else changed."""
+    print(f"append fmt {fmt}:{group} d{d} B{B} Hkv{Hkv} n{n} bt{bt} {order} offset {off}", flush=True)
+    X = hard_rows(B * Hkv, d, group or d, 255 if fmt != R.FMT_INT4 else 15, seed)
+    data, words = quantized(X, fmt, group)
+    # the same as a whole cache: token positions[b] of every head of b (tokens
+    # n..mb * bt - 1 of a paged sequence are in its last page too)
+    mb = -(-n // bt) if bt else 0
+    cap = mb * bt if bt else n
+    at = [(b, h, int(positions[b])) for b in range(B) for h in range(Hkv)]
+    hit = [(i, (b * Hkv + h) * cap + t) for i, (b, h, t) in enumerate(at) if 0 <= t < cap]
+    src, dst = (np.array(v, dtype=np.int64) for v in zip(*hit))
+
+    def whole(rows, fill):
+        out = np.zeros((B * Hkv * cap,) + rows.shape[1:], rows.dtype)
+        out[dst] = rows[src] if fill is None else fill
+        return out
+
+    meta = None if words is None else words.view(np.uint16).reshape(len(X), d // group, 2)
+    want, wmeta, table, _ = O.place(B, Hkv, cap, fmt, group, d, order, bt, whole(data, None),
+                                    None if meta is None else whole(meta, None))
+    used, umeta, _, _ = O.place(B, Hkv, cap, fmt, group, d, order, bt, whole(data, 0xFF),
+                                None if meta is None else whole(meta, 0xFFFF), table=table)
+    keep = []
+    x = _at(keep, 4 * off, torch.float32, X.size)
+    x.copy_(torch.from_numpy(X.reshape(-1).view(np.uint8)))
+    dd = _at(keep, off * (2 if fmt == R.FMT_F16 else 1), torch.uint8, want.size)
+    md = _at(keep, 4 * off, torch.int32, wmeta.size) if wmeta is not None else None
+    tb = torch.from_numpy(table.astype(np.int32)).cuda() if bt else None
+    pos = torch.tensor(positions, dtype=torch.int32, device="cuda:0")
+    R.append_tokens(fmt, group, d, x, B, Hkv, n, pos, order, bt, tb, mb, dd, md)
+    torch.cuda.synchronize()
+    assert np.array_equal(dd.cpu().numpy(), np.where(used == 0xFF, want, 0xA5).reshape(-1).astype(np.uint8))
+    if md is not None:
+        wmeta = np.where(umeta == 0xFFFFFFFF, wmeta, 0xA5A5A5A5).astype(np.uint32)
+        assert np.array_equal(md.cpu().numpy().view(np.uint32), wmeta.reshape(-1))
+    for raw in keep[1:]:
+        assert bool((raw[-64:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("order", [R.ORD_HEAD, R.ORD_TOKEN], ids=["hm", "tm"])
+@pytest.mark.parametrize("fmt,group,d", FORMATS)
+def test_appended_bytes(fmt, group, d, order):
+    # a wave takes 4 (d 128) or 8 (d 64) heads: less than one wave's, one and a
+    # part, several; page sizes that divide by shifting and by division
+    for Hkv in (1, 5, 8, 40):
+        for bt in (0, 12, 16):
+            n = 45
+            past = -(-n // bt) * bt if bt else n
+            positions = [0, n - 1, -1, past - 1, past, 17, 2 ** 31 - 1, -2 ** 31, 31]
+            for off in (0, 1):
+                appended(fmt, group, d, len(positions), Hkv, n, order, bt, off, positions, seed=Hkv + bt)
+
+
+@pytest.mark.parametrize("order,bt", [(R.ORD_HEAD, 0), (R.ORD_TOKEN, 2)])
+def test_appended_bytes_past_a_grid_of_sequences(order, bt):
+    # 65535 sequences are a grid's height; the rest come round again
+    B = 65535 + 70
+    rng = np.random.default_rng(5)
+    appended(R.FMT_INT8, 32, 64, B, 1, 3, order, bt, 0, rng.integers(-1, 5, B), seed=5)
