@@ -1271,8 +1271,9 @@ decode_persistent(uint32_t, uint32_t, const void *, const void *, const void *, 
 //
 // Every workgroup of the head group runs this code once its arrival is
 // counted: the last one on the partials, the others as a dry run (`dry`:
-// zero-length descriptors, so no load reaches memory, one chunk of
-// placeholder splits, and no stores), which brings the code into the XCD's
+// zero-length descriptors, so no load reaches memory, one chunk of as many
+// placeholder splits as the step's first chunk has, so that it runs the same
+// octets, and no stores), which brings the code into the XCD's
 // L2 before the last workgroup fetches it. (Run cold, the code alone takes
 // ~0.85 us of the ~1.8 us merge for GQA 32/8, d128, 32 splits.)
 template <int D, int G, int NW>
@@ -1283,7 +1284,7 @@ __device__ __forceinline__ void merge_heads(const Args &a, const Ext &x, long lo
   constexpr int CPOL = CPOL_SC1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int S = dry ? 1 : a.splits;
+  const int S = dry ? min(a.splits, MCH) : a.splits;
   for (int h = wave; h < G; h += NW) {
     const long long head = head0 + h;
     const __amdgpu_buffer_rsrc_t rml = rsrc(a.part_ml, head * S * 8, dry ? 0u : (uint32_t)(S * 8));
