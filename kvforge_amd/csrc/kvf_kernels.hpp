@@ -164,6 +164,20 @@ template <int FMT, int D, int GQ, int G> struct Geo {
   static constexpr int NCH = ROW / (4 * CH);
   static constexpr int SPC = CH * 8 / BITS / 8;       // MFMA k-steps per chunk
   static constexpr int KSTEPS = NCH * SPC;            // = D / 32
+  // Whether k-step (j, m) holds a dim of one of pass p's groups: with int8:32,
+  // d 128 and 8 heads a chunk j is two groups, one pass's, and the other pass
+  // would multiply zeros and hold them in 32 registers. (With them the 8-wave
+  // kernels reloaded spilled registers at every tile, up to 48 a tile: GQA 64/8,
+  // 16384 tokens of paged rows 34.9 us a step, without 19.2; a batch of 4 of
+  // them 77.7 and 48.9. 4 waves, which spill nothing: 17.0 and 15.5 us for 22541
+  // tokens of contiguous rows.)
+  static constexpr bool qk_used(int p, int j, int m) {
+    for (int r = 0; r < 4; ++r) {
+      const int grp = ((j * 4 * CH + r * CH) * 8 / BITS + 8 * m) / GRP;
+      if (PASSES == 1 || (grp >= p * 16 / G && grp <= (p * 16 + 15) / G)) return true;
+    }
+    return false;
+  }
   // V: lane column c owns dims [c*EV, c*EV+EV) of 8 tokens.
   static constexpr int EV = D / 16;
   static constexpr int VB = EV * BITS / 8;            // bytes per token per lane
@@ -708,6 +722,7 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
     for (int j = 0; j < NCH; ++j)
 #pragma unroll
       for (int m = 0; m < SPC; ++m) {
+        if (!Gm::qk_used(p, j, m)) continue;
         const int ks = j * SPC + m;
         const int dgrp = ((j * 4 * CH + r * CH) * 8 / Gm::BITS + 8 * m) / GRP;
         const float scale = col_live && dgrp == cg ? a.scale_log2 * QPS : 0.f;
@@ -800,10 +815,12 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
           const half8_t av = __builtin_bit_cast(half8_t, (u32x4_t){aw[0], aw[1], aw[2], aw[3]});
           const int ks = j * SPC + m;
 #pragma unroll
-          for (int p = 0; p < PASSES; ++p)
+          for (int p = 0; p < PASSES; ++p) {
+            if (!Gm::qk_used(p, j, m)) continue;
 #pragma unroll
             for (int h2 = 0; h2 < NQ; ++h2)
               cq[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, qb[p][h2][ks], cq[p], 0, 0, 0);
+          }
         }
       }
       static_for<4>([&](auto J) __attribute__((always_inline)) {

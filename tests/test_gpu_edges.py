@@ -47,6 +47,23 @@ def test_every_head_keeps_its_precision(fmt, group, H, Hkv, D):
     assert err < limit(fmt)
 
 
+@pytest.mark.parametrize("fmt", [R.FMT_INT8, R.FMT_INT4])
+@pytest.mark.parametrize("order,bt", [(R.ORD_HEAD, 0), (R.ORD_TOKEN, 16)])
+def test_two_column_passes(fmt, order, bt):
+    # 8 heads by 4 groups: 32 (group, head) columns in two passes. Of int8 rows a
+    # QK step meets one pass's groups and the other leaves it out; of int4 rows
+    # every step meets both. Groups of very different size and sign show a
+    # step that went to the wrong pass.
+    q, K, V = O.make_data(2, 16, 2, 128, 517, 31)
+    K *= np.repeat(np.float32([1, -4, 0.25, 2]), 32)
+    V += np.repeat(np.float32([3, 0, -1, 5]), 32)
+    b = build(Case(2, 16, 2, 128, 517, fmt, 32, order, bt), data=(q, K, V))
+    for splits, warps, unroll in ((1, 4, 2), (1, 8, 4), (3, 8, 2), (5, 4, 4)):
+        err = worst_head(run(b, splits, unroll=unroll, warps=warps), reference(b))
+        print(f"  {b.case.tag()} S{splits} w{warps} u{unroll}: {err:.3g}", flush=True)
+        assert err < limit(fmt)
+
+
 @pytest.mark.parametrize("fmt,group,order,bt", [(R.FMT_F16, 0, R.ORD_HEAD, 0), (R.FMT_INT8, 64, R.ORD_HEAD, 16),
                                                 (R.FMT_INT8, 64, R.ORD_TOKEN, 0), (R.FMT_INT4, 32, R.ORD_TOKEN, 16)])
 def test_tiles_of_a_wave(fmt, group, order, bt):
