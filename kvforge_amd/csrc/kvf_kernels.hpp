@@ -1550,13 +1550,21 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   // of rows) 16.7-17.1 -> 16.2-16.3 us, a paged f16 batch of 4 (75 MB) 17.2 ->
   // 16.6, MHA 4k f16 (67 MB) 15.0 -> 14.8. Below about 1.5 times the L2s' 32 MB
   // it does not (1 MB 6.85 -> 6.90, 4 MB 6.94 -> 7.03, int4 d64 of 34 MB 16.7 ->
-  // 16.9; 38 MB of int8 12.2 -> 12.0), so those keep the plain grid.
-  const double payload = 2.0 * a.B * a.Hkv * (double)a.n * Geo<FMT, D, GQ, G>::ROW;
-  if (fused || (!final_out && !l.partial_only && !x.queue && payload >= 48.0 * (1 << 20))) {
+  // 16.9; 38 MB of int8 12.2 -> 12.0), so those keep the plain grid. Nor does it
+  // for contiguous rows from 144 MiB on in more than two workgroups a CU, whose
+  // rounds of short chunks the plain grid takes in address order (GQA 32/8 of
+  // 300 MiB in 1024 workgroups: f16 55.8 against 53.0 on the plain grid, int8:64
+  // 60.8 and 58.5, int8:32 d64 62.3 and 59.0, int4:32 72.5 and 74.0). Means over
+  // 35 shapes of 768 to 4096 workgroups, affine to plain: 48-100 MiB 0.98, 100-140
+  // MiB 0.99, 160-400 MiB 1.02; paged rows 0.95-1.00 at any size.
+  const double mib = 2.0 * a.B * a.Hkv * (double)a.n * Geo<FMT, D, GQ, G>::ROW / (1 << 20);
+  const bool large = !final_out && !l.partial_only && !x.queue && mib >= 48.0;
+  if (fused || large) {
     DevInfo di;
     const hipError_t e = dev_info(di);
     if (e != hipSuccess) return e;
     const long long nhg = (long long)a.B * gy;
+    const bool rounds = !PAGED && mib >= 144.0 && a.splits * nhg > 2LL * di.cus;
     // (head-major rows only: with token-major rows every KV head sits at one
     // byte offset of each token's row, and one head per XCD made a paged
     // token-major batch of 8 sequences take 38 us fused against 28 us on the
@@ -1568,7 +1576,7 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
     // (splits, heads, B) grid)
     // (a grid holds at most 2^32 - 1 work-items along it, and 65535
     // workgroups in y: larger steps keep the plain grid)
-    if (ORD == ORD_HEAD && !x.seq_lens && di.nx > 1 && di.nx < 16 && nhg % di.nx == 0 && nhg / di.nx <= 65535 &&
+    if (ORD == ORD_HEAD && !x.seq_lens && (fused || !rounds) && di.nx > 1 && di.nx < 16 && nhg % di.nx == 0 && nhg / di.nx <= 65535 &&
         (long long)a.splits * nhg * block.x <= 0xffffffffLL) {
       flags |= (uint32_t)di.nx << KX_NX_SHIFT;
       if (a.B > 1) flags |= KX_HGDIV;

@@ -138,3 +138,98 @@ def test_large_two_launch_steps_on_either_grid(B, Hkv, n):
     R.launch_merge(128, a)
     torch.cuda.synchronize()
     assert worst_head(got, b.out.cpu().numpy().astype(np.float64)) < 1e-5
+
+
+@pytest.mark.parametrize("bt,n,splits", [(0, 9215, 32), (0, 9216, 32), (0, 9216, 8), (16, 9220, 32)])
+def test_large_steps_of_several_rounds(bt, n, splits):
+    # 144 MiB of contiguous rows from n = 9216 on, in more (32 splits) and fewer
+    # than two workgroups a CU; paged rows have no such line. As above.
+    b = build(Case(4, 32, 8, 128, n, R.FMT_F16, 0, R.ORD_HEAD, bt, seed=n), check_cache=False)
+    a = args(b, splits)
+    R.launch(vid(b, True, 2), a)
+    torch.cuda.synchronize()
+    got = b.out.cpu().numpy().copy()
+    b.out.fill_(float("nan"))
+    R.launch_partial(vid(b, True, 2), a)
+    R.launch_merge(128, a)
+    torch.cuda.synchronize()
+    assert worst_head(got, b.out.cpu().numpy().astype(np.float64)) < 1e-5
+
+
+@pytest.mark.parametrize("fmt,group,D,bt,B,Hkv,n,splits", [
+    (R.FMT_F16, 0, 128, 0, 1, 8, 12289, 24), (R.FMT_F16, 0, 128, 16, 4, 8, 3077, 8),
+    (R.FMT_F16, 0, 64, 64, 2, 16, 6200, 5), (R.FMT_INT8, 64, 128, 16, 1, 8, 24577, 32),
+    (R.FMT_INT8, 64, 128, 0, 8, 8, 3103, 16),  # 1024 workgroups: more than are resident at once
+    (R.FMT_INT4, 32, 128, 0, 1, 8, 49155, 32), (R.FMT_INT4, 64, 64, 16, 4, 16, 12301, 8)])
+def test_large_two_launch_steps_against_the_oracle(fmt, group, D, bt, B, Hkv, n, splits):
+    # just past 48 MiB of rows in every format, contiguous and paged
+    b = build(Case(B, 4 * Hkv, Hkv, D, n, fmt, group, R.ORD_HEAD, bt, seed=n), check_cache=False)
+    print(f"  {b.case.tag()} S{splits}", flush=True)
+    ref = O.reference_attention_mt(b.q_host, b.kdeq, b.vdeq, 16)
+    for warps in (4, 8):
+        assert worst_head(run(b, splits, warps=warps), ref) < limit(fmt)
+
+
+@pytest.mark.parametrize("fmt,group,bt", [(R.FMT_INT8, 64, 0), (R.FMT_F16, 0, 16)])
+@pytest.mark.parametrize("n,splits", [(1000, 64), (1003, 8), (40, 3)])
+def test_partials_of_a_whole_step(n, splits, fmt, group, bt):
+    # a whole step's splits are whole tiles, ceil(n / splits) rounded up to 32
+    # tokens: split s holds the attention over its own tokens alone, and the
+    # splits past the end hold (-inf, 0, 0)
+    b = build(Case(2, 8, 2, 128, n, fmt, group, R.ORD_HEAD, bt, seed=n))
+    chunk = -(-(-(-n // splits)) // 32) * 32
+    counters = R.fused_counters(2, 2)
+    for entry in ("two launches", "one launch"):
+        a = args(b, splits)
+        if entry == "one launch":
+            R.launch_fused(vid(b, True, 2), a, counters)
+        else:
+            R.launch(vid(b, True, 2), a)
+        torch.cuda.synchronize()
+        po, pm = (t.cpu().numpy().astype(np.float64) for t in a._keep)
+        for s in range(splits):
+            t0, t1 = min(n, s * chunk), min(n, (s + 1) * chunk)
+            if t0 == t1:
+                assert np.all(np.isneginf(pm[:, :, s, 0])) and not pm[:, :, s, 1].any() and not po[:, :, s].any()
+                continue
+            o, lse, m = O.reference_partials(b.q_host, np.ascontiguousarray(b.kdeq[:, :, t0:t1]),
+                                             np.ascontiguousarray(b.vdeq[:, :, t0:t1]), 1)
+            assert np.max(np.abs(pm[:, :, s, 0] - m[:, :, 0])) < 1e-4
+            assert np.max(np.abs(pm[:, :, s, 0] + np.log2(pm[:, :, s, 1]) - lse[:, :, 0])) < 1e-4
+            assert worst_head(po[:, :, s] / pm[:, :, s, 1:], o[:, :, 0]) < limit(fmt)
+
+
+@pytest.mark.parametrize("D,H,Hkv,splits", [(128, 8, 2, 5), (64, 8, 1, 3), (128, 4, 4, 40)])
+def test_partials_aligned_to_one_float(D, H, Hkv, splits):
+    # part_o and part_ml are floats: buffers that start 4 bytes past a 256-byte
+    # boundary give the same bits, and nothing beside them changes
+    b = build(Case(2, H, Hkv, D, 1500, R.FMT_INT8, 32, R.ORD_HEAD, 0, seed=D + splits))
+    counters = R.fused_counters(2, Hkv)
+    pack = H > Hkv
+
+    def step(entry, off):
+        a = args(b, splits)
+        bufs = []
+        for field, t in zip(("part_o", "part_ml"), a._keep):
+            raw = torch.full((t.numel() + 64,), 7.0, device="cuda:0")
+            bufs.append((raw, t.numel()))
+            setattr(a, field, raw.data_ptr() + 4 * off)
+        b.out.fill_(float("nan"))
+        if entry == "one launch":
+            R.launch_fused(vid(b, pack, 2), a, counters)
+        elif entry == "two launches":
+            R.launch(vid(b, pack, 2), a)
+        else:
+            R.launch_partial(vid(b, pack, 2), a)
+            R.launch_merge(D, a)
+        torch.cuda.synchronize()
+        for raw, size in bufs:
+            assert bool((raw[:off] == 7).all()) and bool((raw[off + size:] == 7).all())
+        return [b.out.cpu().numpy()] + [raw[off:off + size].cpu().numpy() for raw, size in bufs]
+
+    for entry in ("two launches", "one launch", "partial and merge"):
+        want = step(entry, 0)
+        for off in (1, 2, 3):
+            print(f"  D{D} S{splits} {entry} offset {off}", flush=True)
+            for x, y in zip(step(entry, off), want):
+                assert np.array_equal(x, y)
