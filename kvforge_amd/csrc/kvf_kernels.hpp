@@ -845,11 +845,12 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
     // in. Wave-uniform, a branch inside the one body that every tile runs: a
     // body of its own for such tiles made the kernel half as large again and
     // cost copies of the first tile's registers where the two met.
-    if (tbase < t0 || t1 - tbase < TT) {
+    // (The last tile may end past 2^31: those tokens come out negative.)
+    if (tbase < t0 || (uint32_t)tbase + TT > (uint32_t)t1) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const uint32_t t = (uint32_t)tbase + tau(r, i); // (the last tile may end past 2^31)
-        const bool ok = t >= (uint32_t)t0 && t < (uint32_t)t1;
+        const int t = (int)((uint32_t)tbase + tau(r, i));
+        const bool ok = t >= t0 && t < t1;
         s[i] = ok ? s[i] : -INFINITY;
 #pragma unroll
         for (int w = 0; w < VW; ++w) buf.v[i].w[w] = ok ? buf.v[i].w[w] : 0u;
@@ -861,8 +862,8 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       if constexpr (QMETA) {
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
-          const uint32_t t = (uint32_t)tbase + st * SUB + 4 * r + (c & 3); // the lane's word
-          const bool ok = t >= (uint32_t)t0 && t < (uint32_t)t1;
+          const int t = (int)((uint32_t)tbase + st * SUB + 4 * r + (c & 3)); // the lane's word
+          const bool ok = t >= t0 && t < t1;
 #pragma unroll
           for (int p = 0; p < PASSES; ++p) buf.vmr[st].w[p] = ok ? buf.vmr[st].w[p] : 0u;
         }
