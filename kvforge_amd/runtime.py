@@ -185,6 +185,16 @@ def make_args(q, k, v, k_meta, v_meta, table, out, part_o, part_ml, B, H, Hkv, n
 _current_raw = None  # returns the current device's current stream handle
 
 
+def _forget_stream_lookup():
+    global _current_raw
+    _current_raw = None
+
+
+# A forked child of a process that uses the GPU may not: its first call asks
+# torch for the stream again, which refuses.
+os.register_at_fork(after_in_child=_forget_stream_lookup)
+
+
 def stream_handle(stream=None):
     """The hipStream_t of `stream`, or of the current device's current stream
     as it is at this call. The handle is asked for as an integer: a
