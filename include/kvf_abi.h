@@ -38,7 +38,8 @@ struct Args {
   const int *block_table;  /* [B][max_blocks] page ids, paged layouts only */
   float *out;              /* [B][H][D], fp32 */
   float *part_o;           /* [B][H][splits][D] unnormalised partial output */
-  float *part_ml;          /* [B][H][splits][2] running max (log2) and sum */
+  float *part_ml;          /* [B][H][splits][2] running max (log2) and sum; which
+                              tokens a split holds: "Splits" below */
   int B, H, Hkv, n;
   int splits;              /* chunks of the KV length per head */
   int warps;               /* 64-lane wavefronts per workgroup (4 or 8) */
@@ -52,11 +53,7 @@ struct Args {
  * with optional f16 query/output (no counterpart in the reference's Args,
  * which has one n for every sequence and fp32 q/out only,
  * runtime/kvf_kernels.cuh:30-39). Args stays byte-identical; these fields
- * travel beside it. With per-sequence lengths split s of a sequence takes
- * its 32-token tiles s, s + splits, s + 2 * splits, ... (uniform lengths keep
- * the reference's contiguous chunks), so part_o / part_ml hold different
- * partials than a contiguous split would; the merged output agrees to
- * rounding. */
+ * travel beside it. */
 struct VarlenArgs {
   const int *seq_lens;     /* [B] tokens per sequence; Args::n is the maximum */
   const void *q16;         /* [B][H][D] binary16 query, or NULL to use Args::q */
@@ -85,6 +82,19 @@ typedef struct kvf_varlen_args {
   int flags;
 } kvf_varlen_args_t;
 #endif
+
+/* Splits. Split s of a sequence of `len` tokens holds in part_o / part_ml:
+ *   uniform lengths, kvf_launch_partial_variant and its timed forms: the
+ *     reference's chunk, tokens [s * c, min(len, (s + 1) * c)) with
+ *     c = ceil(len / splits) (runtime/kvf_kernels.cuh:147-150);
+ *   uniform lengths, a whole step (every other entry point): the same with c
+ *     rounded up to a multiple of 32;
+ *   per-sequence lengths, contiguous: the same, c rounded up to a multiple of
+ *     32 of the sequence's own length;
+ *   per-sequence lengths, paged: its 32-token tiles s, s + splits,
+ *     s + 2 * splits, ...
+ * A split without tokens holds max -inf, sum 0 and output 0. The merged output
+ * is the same attention to rounding. */
 
 /* Version of this C ABI, also returned by kvf_abi_version(). 2: the one-launch
  * (kvf_launch_fused_variant), persistent and timed-step entry points take
