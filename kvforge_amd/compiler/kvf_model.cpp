@@ -693,13 +693,16 @@ struct CdnaTile {
 
 CdnaTile cdnaTile(const DecodeSpec &s, const Plan &p, int G) {
   CdnaTile t;
-  t.depth = p.part.unroll == 2 ? 2 : 3;
   t.bytes = 32.0 * 2.0 * (p.fmt.dataRowBytes(s.d) + p.fmt.metaRowBytes(s.d));
   const int ng = p.fmt.isQuantized() ? s.d / p.fmt.group : 1;
   const int cols = G * ng;
   const bool hl = cols <= 8; // hi/lo share one MFMA
   const int passes = cols > 16 ? 2 : 1;
   const int nq = hl ? 1 : 2;
+  // 8-wave kernels whose registers do not hold a third tile keep two (depth_of)
+  const int meta_regs = p.fmt.isQuantized() ? (G >= 4 ? 4 : 16) * passes : 0;
+  const int ring3 = 3 * (p.fmt.dataRowBytes(s.d) / 4 + meta_regs) + passes * (nq * (s.d / 32) + s.d / 16) * 4;
+  t.depth = p.part.unroll == 2 || (p.part.warps == 8 && ring3 > 180) ? 2 : 3;
   // QK: 2 sub-tiles x D/32 k-steps x (hi, lo) x passes; PV: D/16 per (hi, lo, pass)
   const double mfma = 2.0 * (s.d / 32) * nq * passes + 1.0 * (s.d / 16) * nq * passes;
   // code -> binary16 conversions per element of K and V, softmax per token slot

@@ -43,11 +43,11 @@
 //
 // Streaming: every wave keeps a ring of DEPTH tiles; tile k+DEPTH-1 is
 // issued before tile k is consumed. Loads are raw buffer loads through
-// per-sub-tile descriptors built in scalar registers: the record count
-// stops the loads at the sequence end, and a tile outside the wave's range
-// gets zero-length descriptors whose loads return zeros without touching
-// memory, so the load stream is unconditional and the compiler's wait counts
-// are static. Within a tile both sub-tiles' K go first, then the (scale,
+// descriptors in scalar registers, one over the tile for contiguous rows and
+// one a sub-tile for paged ones: the record count stops the loads at the end of
+// the split's range, and a tile outside it gets zero-length descriptors whose
+// loads return zeros without touching memory, so the load stream is
+// unconditional and the compiler's wait counts are static. Within a tile both sub-tiles' K go first, then the (scale,
 // zero) words, then V, so scores and softmax start before V has arrived.
 // The first DEPTH-1 tiles are issued before the query is converted, so the
 // two latencies overlap. Head-major rows load as nontemporal; token-major
@@ -146,9 +146,6 @@ template <int D, int G> constexpr bool hl_lds_fits(int nw) {
 }
 template <int FMT, int D, int GQ, int G> constexpr size_t combine_lds(int nw);
 
-// Tiles kept in flight per wave for the reference's unroll knob U.
-template <int U> constexpr int depth_of() { return U == 2 ? 2 : 3; }
-
 // Lane geometry of one (format, head dim, quantisation group, pack size).
 template <int FMT, int D, int GQ, int G> struct Geo {
   static constexpr int BITS = bits_of<FMT>();
@@ -185,6 +182,10 @@ template <int FMT, int D, int GQ, int G> struct Geo {
   // G >= 4: the 4 columns of a quad share a group, so lane (r, c) loads the
   // whole meta row of token 4r + c%4 and a quad broadcast hands it around
   static constexpr bool QMETA = QUANT && G >= 4;
+  // Registers that a wave holds through the loop with a ring of three tiles:
+  // the tiles, the query operands and the accumulators.
+  static constexpr int TILE_REGS = ROW / 4 + (QUANT ? (QMETA ? 4 : 16) * PASSES : 0);
+  static constexpr int RING3_REGS = 3 * TILE_REGS + PASSES * (HL ? 1 : 2) * KSTEPS * 4 + PASSES * EV * 4;
   static_assert(D == 64 || D == 128, "head dimension");
   static_assert(G == 1 || G == 2 || G == 4 || G == 8, "pack size");
   static_assert(KSTEPS * 32 == D, "chunk geometry");
@@ -192,6 +193,19 @@ template <int FMT, int D, int GQ, int G> struct Geo {
   static_assert(!QUANT || (GQ >= 32 && GQ <= D), "group");
   static_assert(COLS <= 32, "at most two column passes");
 };
+
+// Tiles kept in flight per wave for the reference's unroll knob U: 2, or 3. A
+// wave of eight has 256 registers, which three tiles of some formats do not fit
+// beside the 75 or so that the rest takes (at 172 counted ones the kernels take
+// 247, at 192 they spill). A spilled register's reload waits for every load in
+// flight, so those kernels keep two tiles: d 128 in f16, int8 with 1 or 2 heads,
+// and either of int8:32 and int4:32 with 8. Over their 2016 plans of a sweep of
+// 12 shapes two tiles take 0.76 of the time of three (median; 0.40 to 1.06, by
+// kernel 0.57 to 0.95), e.g. GQA 32/8 int8:128 unpacked, 65536 token-major
+// tokens in one split, 844 -> 517 us.
+template <int U, int WPB, class Gm> constexpr int depth_of() {
+  return U == 2 || (WPB == 8 && Gm::RING3_REGS > 180) ? 2 : 3;
+}
 
 template <int FMT, int D, int GQ, int G> constexpr size_t combine_lds(int nw) {
   const bool sl = Geo<FMT, D, GQ, G>::HL && hl_lds_fits<D, G>(nw);
@@ -376,7 +390,6 @@ template <int N, int I = 0, class F> __device__ __forceinline__ void static_for(
 __device__ __forceinline__ int tau(int r, int i) { return (i >> 2) * SUB + 4 * r + (i & 3); }
 
 constexpr int CPOL_SC1 = 16; // buffer-load cache policy: device-coherent (sc1)
-constexpr int CPOL_SC0 = 1;  // buffer-load cache policy: skip the CU's L1, served by L2
 template <int D, int G, int NW>
 __device__ __forceinline__ void merge_heads(const Args &a, const Ext &x, long long head0, bool dry);
 
@@ -420,7 +433,7 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
   constexpr int ROW = Gm::ROW, NG = Gm::NG, COLS = Gm::COLS, PASSES = Gm::PASSES;
   constexpr int CH = Gm::CH, NCH = Gm::NCH, SPC = Gm::SPC, KSTEPS = Gm::KSTEPS;
   constexpr int EV = Gm::EV, VB = Gm::VB, VW = Gm::VW, GRP = Gm::GRP;
-  constexpr int DEPTH = depth_of<U>();
+  constexpr int DEPTH = depth_of<U, WPB, Gm>();
   constexpr bool HL_LDS = HL && hl_lds_fits<D, G>(WPB);
   constexpr int NQ = HL ? 1 : 2;                   // query operands per k-step
   constexpr float UNIT = QUANT ? SUB_UNIT / Q_PRESCALE : 1.f; // log2 units per score unit
