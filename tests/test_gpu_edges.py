@@ -10,7 +10,7 @@ are fp32: per head the steps measure up to 5e-6 (int8 with outlier channels),
 2e-6 (f16) and 3e-5 (int4:32, whose scales are 17 times larger). A pair whose
 halves do not belong together is off by a binary16 ulp of one element, 2^-11
 of its share of a score: 7e-5 to 6e-4 of a head. So heads are held to 2^-15
-(int8, f16), and int4 to 2^-13."""
+(int8, f16), and int4 to 2^-14, twice what it measures and below 7e-5."""
 import numpy as np
 import pytest
 import torch
@@ -35,10 +35,11 @@ def worst_head(got, ref):
 
 
 def limit(fmt):
-    return 2.0 ** -13 if fmt == R.FMT_INT4 else 2.0 ** -15
+    return 2.0 ** -14 if fmt == R.FMT_INT4 else 2.0 ** -15
 
 
-@pytest.mark.parametrize("fmt,group", [(R.FMT_F16, 0), (R.FMT_INT8, 64), (R.FMT_INT8, 32)])
+@pytest.mark.parametrize("fmt,group", [(R.FMT_F16, 0), (R.FMT_INT8, 64), (R.FMT_INT8, 32), (R.FMT_INT4, 32),
+                                       (R.FMT_INT4, 64)])
 @pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (16, 16, 64), (32, 4, 64)])
 def test_every_head_keeps_its_precision(fmt, group, H, Hkv, D):
     b = build(Case(16, H, Hkv, D, 64, fmt, group, R.ORD_HEAD, 0, seed=3, outliers=True))
@@ -70,8 +71,9 @@ def test_tiles_of_a_wave(fmt, group, order, bt):
     for n in (1, 31, 33, 127, 128, 160, 257, 385, 641, 1003):
         b = build(Case(1, 8, 2, 128, n, fmt, group, order, bt, seed=n))
         for splits, warps, unroll in ((1, 4, 2), (1, 8, 4), (3, 4, 2), (8, 4, 4), (16, 8, 2)):
-            print(f"  {b.case.tag()} S{splits} w{warps} u{unroll}", flush=True)
-            assert worst_head(run(b, splits, unroll=unroll, warps=warps), reference(b)) < limit(fmt)
+            err = worst_head(run(b, splits, unroll=unroll, warps=warps), reference(b))
+            print(f"  {b.case.tag()} S{splits} w{warps} u{unroll}: worst head {err:.3g}", flush=True)
+            assert err < limit(fmt)
 
 
 @pytest.mark.parametrize("B,H,Hkv", [(1, 32, 8), (4, 8, 2), (3, 64, 16), (2, 16, 16)])
@@ -119,7 +121,9 @@ def test_unequal_lengths(fmt, group, order, bt):
         torch.cuda.synchronize()
         got = b.out.cpu().numpy()
         assert not got[1].any()
-        assert worst_head(got, ref) < limit(fmt)
+        err = worst_head(got, ref)
+        print(f"  {b.case.tag()} lengths S{splits}: worst head {err:.3g}", flush=True)
+        assert err < limit(fmt)
 
 
 @pytest.mark.parametrize("B,Hkv,n", [(1, 8, 24575), (1, 8, 24576), (2, 4, 24601), (1, 3, 65536)])
@@ -167,7 +171,9 @@ def test_large_two_launch_steps_against_the_oracle(fmt, group, D, bt, B, Hkv, n,
     print(f"  {b.case.tag()} S{splits}", flush=True)
     ref = O.reference_attention_mt(b.q_host, b.kdeq, b.vdeq, 16)
     for warps in (4, 8):
-        assert worst_head(run(b, splits, warps=warps), ref) < limit(fmt)
+        err = worst_head(run(b, splits, warps=warps), ref)
+        print(f"  {b.case.tag()} w{warps}: worst head {err:.3g}", flush=True)
+        assert err < limit(fmt)
 
 
 @pytest.mark.parametrize("fmt,group,bt", [(R.FMT_INT8, 64, 0), (R.FMT_F16, 0, 16)])
