@@ -1572,7 +1572,12 @@ hipError_t launch_group(const Args &a, const Ext &x, const Launch &l, hipStream_
   // 35 shapes of 768 to 4096 workgroups, affine to plain: 48-100 MiB 0.98, 100-140
   // MiB 0.99, 160-400 MiB 1.02; paged rows 0.95-1.00 at any size.
   const double mib = 2.0 * a.B * a.Hkv * (double)a.n * Geo<FMT, D, GQ, G>::ROW / (1 << 20);
-  const bool large = !final_out && !l.partial_only && !x.queue && mib >= 48.0;
+  // (Query heads that share a KV head without packing read its rows through
+  // one XCD's L2 on the plain grid, whose XCD follows the split; one XCD a head
+  // reads them from memory once a head: 32 heads on 8 KV heads in 8 splits, 65536
+  // tokens of int8:64 97.7 us affine and 76.1 plain, with 8 waves 140 and 88.9,
+  // 32768 tokens of paged f16 90.5 and 65.2.)
+  const bool large = !final_out && !l.partial_only && !x.queue && (G > 1 || a.H == a.Hkv) && mib >= 48.0;
   if (fused || large) {
     DevInfo di;
     const hipError_t e = dev_info(di);

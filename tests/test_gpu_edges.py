@@ -239,3 +239,13 @@ def test_partials_aligned_to_one_float(D, H, Hkv, splits):
             print(f"  D{D} S{splits} {entry} offset {off}", flush=True)
             for x, y in zip(step(entry, off), want):
                 assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("fmt,group,D,bt,n", [(R.FMT_F16, 0, 128, 16, 12300), (R.FMT_INT8, 64, 128, 0, 24600)])
+def test_large_steps_of_unpacked_query_heads(fmt, group, D, bt, n):
+    # past 48 MiB of rows, four query heads a KV head without packing: the plain
+    # grid, against the oracle
+    b = build(Case(1, 32, 8, D, n, fmt, group, R.ORD_HEAD, bt, seed=n), check_cache=False)
+    ref = O.reference_attention_mt(b.q_host, b.kdeq, b.vdeq, 16)
+    for splits in (4, 8):
+        assert worst_head(run(b, splits, pack=False), ref) < limit(fmt)
