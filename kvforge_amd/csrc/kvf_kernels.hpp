@@ -636,6 +636,10 @@ __device__ __forceinline__ void decode_item(const Args &a, const Ext &x, const i
       }
       sub_k = SUB * (int)row_step;
       sub_m = SUB * (int)meta_step;
+      // two column passes in 8 waves have no registers for the second
+      // sub-tile's offsets: worked out anew for every tile (int4:32 with 8 heads,
+      // 8192 tokens, 1 and 4 splits: 91 -> 66 and 31.4 -> 25.0 us)
+      if constexpr (ORD == ORD_TOKEN && PASSES == 2 && WPB == 8) asm("" : "+s"(sub_k), "+s"(sub_m) : "s"(left));
     } else {
       if ((knext & 31) == 0 && knext > 0) {
         load_pages(knext);

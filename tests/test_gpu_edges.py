@@ -49,7 +49,7 @@ def test_every_head_keeps_its_precision(fmt, group, H, Hkv, D):
 
 
 @pytest.mark.parametrize("fmt", [R.FMT_INT8, R.FMT_INT4])
-@pytest.mark.parametrize("order,bt", [(R.ORD_HEAD, 0), (R.ORD_TOKEN, 16)])
+@pytest.mark.parametrize("order,bt", [(R.ORD_HEAD, 0), (R.ORD_TOKEN, 0), (R.ORD_TOKEN, 16)])
 def test_two_column_passes(fmt, order, bt):
     # 8 heads by 4 groups: 32 (group, head) columns in two passes. Of int8 rows a
     # QK step meets one pass's groups and the other leaves it out; of int4 rows
