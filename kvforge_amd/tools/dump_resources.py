@@ -16,16 +16,19 @@ token-major 1); `group` is the quantisation group the kernel is built for (the
 head dimension for f16), `g` the GQA pack, `u` the unroll knob, `waves` the
 wavefronts per workgroup; `occupancy` is the compiler's waves per SIMD.
 
-valu, mfma, lds, salu: instructions per 32-token tile of the kernel's main
-loop, counted in the gfx950 assembly of the same compile (-S): the loop is
-the one holding the most MFMAs in its own blocks (the main loop comes in a
-masked and an unmasked copy, one for chunks that start inside a tile; the
-unmasked one, with fewer vector instructions, is taken); its blocks hold the
-tile's compute once per unrolled step, so the counts are divided by (MFMAs
-in the loop / MFMAs per tile). MFMAs per
+valu, mfma, lds, salu: instructions that every 32-token tile of the kernel's
+main loop runs, counted in the gfx950 assembly of the same compile (-S): the
+loop is the one holding the most MFMAs in its own blocks. Of its blocks only
+those count that every iteration passes through: the masking of a tile that
+reaches outside the split's range, the rescaling when a score passes the
+running max, and the next page ids of paged rows are behind wave-uniform
+branches that a tile rarely takes. The blocks hold the tile's compute once per
+unrolled step, so the counts are divided by (MFMAs in the loop / MFMAs per
+tile). MFMAs per
 tile follow from the kernel's column geometry: COLS = g x (d / group) query
 columns (g for f16), two passes when COLS > 16, hi and lo in one MFMA when
-COLS <= 8, and per pass and binary16 half 2 x d/32 QK steps plus d/16 PV
+COLS <= 8, and per pass and binary16 half 2 x d/32 QK steps (of int8:32 at d
+128 and 8 heads only the half that meets the pass's groups) plus d/16 PV
 steps. `lds` counts ds_* instructions (the cross-row shuffles), `salu` s_*.
 """
 import argparse
@@ -54,29 +57,60 @@ LABEL = re.compile(r"^(_Z\w+):")
 BLOCK = re.compile(r"^(\.LBB\d+_\d+):(.*)")
 BB = re.compile(r"^; (%bb\.\d+):(.*)")
 IN_LOOP = re.compile(r"Header=BB(\d+_\d+) Depth=\d+")
+BRANCH = re.compile(r"(s_cbranch_\w+|s_branch)\s+(\.LBB\d+_\d+)")
 
 
 def mfma_per_tile(fmt, d, group, g):
     cols = g * (d // group if fmt != 0 else 1)
     passes = 2 if cols > 16 else 1
     nq = 1 if cols <= 8 else 2
-    return (2 * (d // 32) + d // 16) * nq * passes
+    # int8:32, d 128, 8 heads: a QK step holds dims of one pass's groups only
+    qk_passes = 1 if (fmt, d, group, g) == (1, 128, 32, 8) else passes
+    return (2 * (d // 32) * qk_passes + d // 16 * passes) * nq
+
+
+def every_iteration(header, body, order, targets, falls):
+    """The blocks of `body` that lie on every path from `header` back to it (all
+    of them, if no branch leads back). `order` is the function's blocks as laid
+    out, targets[b] where b's branches go, falls[b] whether b runs on into the
+    next block."""
+    body = set(body)
+    after = dict(zip(order, order[1:]))
+
+    def comes_round(without):
+        seen, todo = set(), [header]
+        while todo:
+            b = todo.pop()
+            if b in seen or b == without:
+                continue
+            seen.add(b)
+            for t in targets[b] + ([after[b]] if falls[b] and b in after else []):
+                if t == header:
+                    return True
+                if t in body:
+                    todo.append(t)
+        return False
+
+    if not comes_round(None):
+        return body
+    return {b for b in body if b == header or not comes_round(b)}
 
 
 def loop_mix(lines):
     """Instruction mix of the loop with the most MFMAs in its own blocks (the
-    fewest vector instructions breaking a tie). A
+    fewest vector instructions breaking a tie), over the blocks that every
+    iteration runs. A
     block (a `.LBB` label or an unlabelled `; %bb.N:` fall-through) counts for
     the innermost loop holding it, as the assembler's comments on the block's
     first lines name it ("Loop Header: Depth=d" for a header, "in Loop:
     Header=BBx_y" for the others)."""
-    blocks, notes, order = {}, {}, []
+    blocks, notes, order, targets = {}, {}, [], {}
     cur, head = None, False
     for line in lines:
         m = BLOCK.match(line) or BB.match(line)
         if m:
             cur = m.group(1)
-            blocks[cur], notes[cur], head = [], m.group(2), True
+            blocks[cur], notes[cur], targets[cur], head = [], m.group(2), [], True
             order.append(cur)
             continue
         t = line.strip()
@@ -89,6 +123,9 @@ def loop_mix(lines):
         head = False
         if t[0] != ".":
             blocks[cur].append(t.split()[0])
+            if (m := BRANCH.match(t)):
+                targets[cur].append(m.group(2))
+    falls = {b: not (ops and ops[-1] in ("s_branch", "s_endpgm", "s_setpc_b64")) for b, ops in blocks.items()}
     loops = {}
     for b in order:
         if "Loop Header: Depth=" in notes[b]:
@@ -97,14 +134,16 @@ def loop_mix(lines):
             h = IN_LOOP.search(notes[b])
             owner = "BB" + h.group(1) if h else None
         if owner:
-            loops.setdefault(owner, []).extend(blocks[b])
+            loops.setdefault(owner, []).append(b)
     if not loops:
         return None
-    # of several loops with that many MFMAs (the main loop's masked and
-    # unmasked copies), the one with the fewest vector ALU instructions: the
-    # unmasked copy, which every chunk starting on a tile boundary runs
-    ops = max(loops.values(), key=lambda o: (sum(x.startswith("v_mfma") for x in o),
-                                             -sum(x.startswith("v_") for x in o)))
+
+    def ops_of(body):
+        return [x for b in body for x in blocks[b]]
+
+    body = max(loops.values(), key=lambda bs: (sum(x.startswith("v_mfma") for x in ops_of(bs)),
+                                               -sum(x.startswith("v_") for x in ops_of(bs))))
+    ops = ops_of(every_iteration(body[0], body, order, targets, falls))
     mix = {"mfma": 0, "valu": 0, "lds": 0, "salu": 0}
     for op in ops:
         if op.startswith("v_mfma"):

@@ -274,11 +274,10 @@ def test_mi355x_model_top1_against_measured_sweep(tmp_path):
     # the committed constants against the committed MI355X sweep (every plan of
     # 12 uniform shapes timed on the GPU with the kernels of the same commit):
     # with every format allowed the model's top-1 is on average within 4 % of
-    # the measured best and never 9 % away (the worst is the 14 us MHA d64
-    # batch-2 shape at 8.0 %, where unroll 4 is ranked above unroll 2; the next
-    # two are 7.5 and 5.9 %); among f16 and int8 plans the mean is 0.6 % and the
-    # worst 2.3 %; and the north star's int8:64 pick is the measured best (the
-    # north star asks for 10 %)
+    # the measured best and never 9 % away (1.9 %; the worst is the 13 us MHA d64
+    # batch-2 shape at 8.5 %, the next 2.7 %); among f16 and int8 plans the mean
+    # is 0.3 % and the worst 1.6 %; and the north star's int8:64 pick is the
+    # measured best (the north star asks for 10 %)
     text = _evaluate(tmp_path, "--which", "all")
     blk = _block(text, "no accuracy limit")
     regret_max = float(blk.split("regret max")[1].split("%")[0])
@@ -302,9 +301,9 @@ def test_mi355x_model_on_the_mixed_shape_sweep(tmp_path):
     # the mixed-shape sweep (every plan of the log-uniform GQA 64/8 B16 batch,
     # of GQA-4 d64 B4 and of config 3's paged batch, timed on the GPU with
     # their own per-sequence lengths): the committed constants pick config 3's
-    # measured best; every f16 and int8 pick is the measured best, and with
+    # measured best; every f16 and int8 pick is within 0.9 % of it, and with
     # int4 allowed the worst is the log-uniform batch's int4:128 pick with
-    # unroll 4 ranked above unroll 2 (10.8 %)
+    # unroll 4 ranked above unroll 2 (8.9 %)
     sweep = tmp_path / "mixed.csv"
     with gzip.open(os.path.join(ROOT, "kvforge_amd", "model", "sweep_mixed_mi355x.csv.gz"), "rb") as f:
         sweep.write_bytes(f.read())
@@ -325,7 +324,8 @@ def test_mi355x_model_on_the_mixed_shape_sweep(tmp_path):
 
 def test_mi355x_model_on_the_head_share_sweep(tmp_path):
     # every plan (splits up to 256) of one GPU's share of GQA 32/8 d128 at 32k
-    # tokens when 2, 4 or 8 GPUs split the KV heads, timed on the GPU: the
+    # tokens when 2, 4 or 8 GPUs split the KV heads, timed on the GPU (with the
+    # kernels before the one-body loop): the
     # committed constants stay within 6 % of the measured best in every
     # accuracy class, and pick a split count that fills the chip as the
     # measured best does (64 for 4 KV heads, 128 for 2, 128 or 256 for 1: the

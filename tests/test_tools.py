@@ -58,6 +58,44 @@ def test_loop_mix_takes_the_unmasked_copy():
     assert mix["mfma"] == 16 and mix["valu"] == 400, mix
 
 
+def test_loop_mix_leaves_out_what_a_tile_rarely_runs():
+    # one loop of two steps: in each, a masking block that a branch skips and a
+    # rescaling block placed out of line, which branches back
+    mfma, add, mask, rescale = "v_mfma_f32_16x16x32_f16", "v_add_f32", "v_cndmask_b32", "v_mul_f32"
+
+    def block(label, ops, branches=()):
+        return [f"{label}: ;   in Loop: Header=BB0_1 Depth=1"] + [f"\t{op} v0, v1" for op in ops] + \
+               [f"\t{op} {to}" for op, to in branches]
+
+    lines = ["; %bb.0:", "\ts_nop 0"]
+    lines += [".LBB0_1: ; =>This Inner Loop Header: Depth=1"] + [f"\t{op} v0, v1" for op in [mfma] * 4 + [add] * 10] + \
+             ["\ts_cbranch_vccnz .LBB0_3"]
+    lines += block("; %bb.2", [mask] * 7)
+    lines += block(".LBB0_3", [add] * 3, [("s_cbranch_vccz", ".LBB0_8")])
+    lines += block(".LBB0_4", [mfma] * 4 + [add] * 10, [("s_cbranch_vccnz", ".LBB0_6")])
+    lines += block("; %bb.5", [mask] * 7)
+    lines += block(".LBB0_6", [add] * 3, [("s_cbranch_scc0", ".LBB0_9")])
+    lines += block("; %bb.7", ["s_add_u32"], [("s_branch", ".LBB0_1")])
+    lines += block(".LBB0_8", [rescale] * 20, [("s_branch", ".LBB0_4")])
+    lines += [".LBB0_9:", "\ts_endpgm"]
+    mix = dump_resources.loop_mix(lines)
+    assert mix["mfma"] == 8 and mix["valu"] == 26 and mix["lds"] == 0, mix
+    assert mix["salu"] == 6, mix  # five branches and the add
+
+
+def test_spilling_kernels_are_the_two_pass_ones():
+    # a spilled register's reload waits behind every load in flight: the table
+    # of the compiled kernels has scratch only where two column passes meet 8
+    # waves, and little of it
+    import csv
+    with open(os.path.join(ROOT, "machines", "resources_gfx950.csv")) as f:
+        rows = list(csv.DictReader(f))
+    assert len(rows) == 768
+    for r in rows:
+        if int(r["scratch"]):
+            assert (r["d"], r["group"], r["g"], r["waves"]) == ("128", "32", "8", "8") and int(r["scratch"]) <= 72, r
+
+
 def test_mfma_per_tile_follows_the_column_geometry():
     # f16 d128 (COLS = g): 2 x 4 QK steps + 8 PV steps per pass and half
     assert dump_resources.mfma_per_tile(0, 128, 0, 4) == 16
