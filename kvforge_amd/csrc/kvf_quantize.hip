@@ -155,9 +155,9 @@ __device__ __forceinline__ void put_row(f4u v0, f4u v1, int c, long long prow, u
 // takes 62.3); the codes' stores are nontemporal, the rows' loads are not (they
 // are often still cached: with nontemporal loads 8000 tokens 16.8 -> 18.5 us).
 // Measured on MI355X, K and V of one layer with 8 KV heads of 128: 32768
-// tokens in int8:64, head-major contiguous, 339 -> 62 us (5.5 TB/s read and
-// written; a large copy reaches 5.2); 4 x 4093 tokens in int4:32, paged
-// token-major, 180 -> 35 us (4.4 TB/s). Before, a wave took one row, a lane
+// tokens in int8:64, head-major contiguous, 339 -> 59 us (5.8 TB/s read and
+// written; a large copy reaches 5.3); 4 x 4093 tokens in int4:32, paged
+// token-major, 180 -> 32 us (4.9 TB/s). Before, a wave took one row, a lane
 // single elements with byte stores, and every element one division.
 template <int FMT, int D, int GQ>
 __global__ void __launch_bounds__(256)
