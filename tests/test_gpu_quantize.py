@@ -188,3 +188,37 @@ def test_appended_bytes_past_a_grid_of_sequences(order, bt):
     B = 65535 + 70
     rng = np.random.default_rng(5)
     appended(R.FMT_INT8, 32, 64, B, 1, 3, order, bt, 0, rng.integers(-1, 5, B), seed=5)
+
+
+@pytest.mark.parametrize("fmt,group,d", [f for f in FORMATS if f[1]])
+def test_signalling_nans_are_skipped(fmt, group, d):
+    # one signalling NaN of either sign at every place of a group, beside the
+    # group's minimum and maximum at every other place: both stay
+    rng = np.random.default_rng(group)
+    n = 4 * group
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    for r in range(n):
+        g = X[r].reshape(-1, group)
+        for i in range(len(g)):
+            lo, hi, nan = rng.permutation(group)[:3]
+            nan = r % group
+            lo, hi = ((v + 1) % group if v == nan else v for v in (lo, hi))
+            g[i, lo], g[i, hi] = -9.0 - i, 11.0 + i
+            g[i].view(np.uint32)[nan] = 0x7F9CC28F if (r // group) % 2 else 0xFFA6D5A5
+    # (numpy's own minimum loses its neighbour to a signalling NaN in one
+    # dimension: the restatement gets them quiet, which it skips everywhere)
+    quiet = np.where(np.isnan(X), np.float32(np.nan), X)
+    data, words = quantized(quiet, fmt, group)
+    for entry in ("place", "append"):
+        B, Hkv = (1, 1) if entry == "place" else (n // 4, 4)
+        x = torch.from_numpy(X.view(np.int32)).cuda()
+        dd = torch.zeros(data.size, dtype=torch.uint8, device="cuda:0")
+        md = torch.zeros(words.size, dtype=torch.int32, device="cuda:0")
+        if entry == "place":
+            R.quantize_place(fmt, group, d, x, B, Hkv, n, R.ORD_HEAD, 0, None, 0, dd, md)
+        else:
+            R.append_tokens(fmt, group, d, x, B, Hkv, 1, torch.zeros(B, dtype=torch.int32, device="cuda:0"), R.ORD_HEAD, 0,
+                            None, 0, dd, md)
+        torch.cuda.synchronize()
+        assert np.array_equal(md.cpu().numpy().view(np.uint32), words.reshape(-1)), entry
+        assert np.array_equal(dd.cpu().numpy(), data.reshape(-1)), entry
